@@ -827,3 +827,35 @@ def test_layer_norm_fp32_to_fp16_is_the_rounded_fp32_result(gpu, K):
     y16 = ops.layer_norm(xg, wg, bg, 1e-5, out_dtype=torch.float16)
     assert y16.dtype == torch.float16
     assert torch.equal(y16, y32.half())
+
+
+# --------------------------------------------------------------- K that fills no whole step
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,N", [(4100, 4360), (1100, 3000), (600, 1100)])
+@pytest.mark.parametrize("K", [8, 72, 184])
+def test_linear_ragged_k(gpu, dtype, M, N, K):
+    """The LDS-DMA loader's last, partly filled step at every tile size (256, 128, 64), with a
+    row-strided A whose bytes past K are NaN: they must read as zeros."""
+    ops = _ops()
+    a = torch.full((M, K + 24), float("nan"), dtype=dtype)
+    a[:, :K] = _rand((M, K), dtype, 1)
+    w = _rand((N, K), dtype, 2, scale=K ** -0.5)
+    b = _rand((N,), torch.float32, 3, scale=0.1)
+    print(f"ragged K dtype={dtype} M={M} N={N} K={K}", flush=True)
+    out = ops.linear(a.to(gpu)[:, :K], w.to(gpu), b.to(gpu)).cpu().double()
+    a64, w64 = a[:, :K].double(), w.double()
+    ref = a64 @ w64.T + b.double()
+    bound = UNIT[dtype] * ref.abs() + 4 * K * 2.0 ** -24 * (a64.abs() @ w64.abs().T) + 1e-7
+    assert _report("linear", (out - ref).abs(), bound) <= 1.0
+
+
+@pytest.mark.parametrize("M,N,K", [(2100, 1100, 16), (4100, 4360, 144), (1100, 3000, 272)])
+def test_gemm_i8_ragged_k_bit_exact(gpu, M, N, K):
+    ops = _ops()
+    rng = np.random.default_rng(M + N + K)
+    a = rng.integers(-128, 128, size=(M, K), dtype=np.int8)
+    w = rng.integers(-128, 128, size=(N, K), dtype=np.int8)
+    acc = torch.empty(M, N, dtype=torch.int32, device=gpu)
+    ops.linear_i8(torch.from_numpy(a).to(gpu), torch.from_numpy(w).to(gpu),
+                  torch.ones(M, device=gpu), torch.ones(N, device=gpu), acc_out=acc, want_out=False)
+    np.testing.assert_array_equal(acc.cpu().numpy(), OI.int8_gemm(a, w))

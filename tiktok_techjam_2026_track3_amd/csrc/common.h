@@ -86,6 +86,40 @@ struct Mfma<float> {
   }
 };
 
+// The 16x16 MFMA family of the projection GEMMs: operand fragments as above, a 16-byte chunk per
+// lane (row l % 16, chunk l / 16 of four), accumulator 4 values per lane: lane l, register i holds
+// D[m][n] with n = l % 16, m = 4 * (l / 16) + i.
+template <typename T>
+struct Mfma16;
+
+template <>
+struct Mfma16<_Float16> {
+  using frag = f16x8;
+  using acc = f32x4;
+  static constexpr int ELEMS_PER_CHUNK = 8;
+};
+
+template <>
+struct Mfma16<__bf16> {
+  using frag = bf16x8;
+  using acc = f32x4;
+  static constexpr int ELEMS_PER_CHUNK = 8;
+};
+
+template <>
+struct Mfma16<int8_t> {
+  using frag = i32x4;
+  using acc = i32x4;
+  static constexpr int ELEMS_PER_CHUNK = 16;
+};
+
+template <>
+struct Mfma16<float> {
+  using frag = f32x4;  // 4 x fp32, consumed one element per MFMA (16x16x4)
+  using acc = f32x4;
+  static constexpr int ELEMS_PER_CHUNK = 4;
+};
+
 // Accumulator layout of the 32x32 MFMAs (D = A·B, A rows = m, B columns = n):
 // lane l, register i holds D[m][n] with n = l % 32 and m = 8*(i/4) + 4*(l/32) + (i%4).
 // Operand layout: lane l supplies A[m = l%32][k-slice (l/32)] and B[k-slice (l/32)][n = l%32];
@@ -150,6 +184,20 @@ MI355_DEVINL void buffer_dma_lds16(u32x4 rsrc, uint32_t voffset, uint32_t soffse
                "s"(rsrc), "s"(__builtin_amdgcn_readfirstlane(soffset)),
                "s"(__builtin_amdgcn_readfirstlane(lds_addr))
                : "memory", "m0");
+}
+// The same from rsrc base + voffset + vstep + soffset with a wave-uniform vstep, added to the
+// lane's offset here so that the sum takes part in the range check and is not kept in a register,
+// to LDS lds_addr + LDS_STEP + 16 lane (the VALU add is the wait state between M0 and the load).
+template <int LDS_STEP = 0>
+MI355_DEVINL void buffer_dma_lds16(u32x4 rsrc, uint32_t voffset, uint32_t vstep, uint32_t soffset,
+                                   uint32_t lds_addr) {
+  uint32_t sum;
+  asm volatile("s_add_u32 m0, %4, %6\n\tv_add_u32 %0, %5, %1\n\tbuffer_load_dwordx4 %0, %2, %3 offen lds"
+               : "=&v"(sum)
+               : "v"(voffset), "s"(rsrc), "s"(__builtin_amdgcn_readfirstlane(soffset)),
+                 "s"(__builtin_amdgcn_readfirstlane(lds_addr)),
+                 "s"(__builtin_amdgcn_readfirstlane(vstep)), "i"(LDS_STEP)
+               : "memory", "m0", "scc");
 }
 MI355_DEVINL float pair_sum(float v) {
   auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
