@@ -829,6 +829,48 @@ def test_layer_norm_fp32_to_fp16_is_the_rounded_fp32_result(gpu, K):
     assert torch.equal(y16, y32.half())
 
 
+# ------------------------------------------------- tiled 16-bit attention at the other head dims
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("hd", [8, 16, 48, 80, 96, 192, 256])
+@pytest.mark.parametrize("B,Sq,Sk,H", [
+    (1, 8, 8, 3), (1, 9, 9, 3),          # the vector-ALU kernel's last size (192, 256) and the next
+    (2, 32, 32, 2), (2, 32, 33, 2),      # one 32-key tile; two tiles
+    (1, 33, 65, 2), (2, 128, 128, 1),    # 128-query work-groups, their last size
+    (1, 129, 192, 2), (130, 260, 70, 2),  # too few 256-query work-groups; enough of them
+])
+def test_attention_tiled_edges(gpu, dtype, hd, B, Sq, Sk, H):
+    """Edges of the work-group and key tiles of attn_fwd_tiled, with and without a key mask."""
+    if B > 4:
+        B = B if hd <= 96 else 66
+    kv = torch.ones(B, Sk, dtype=torch.bool)
+    kv[:, Sk // 2:] = torch.rand(B, Sk - Sk // 2, generator=torch.Generator().manual_seed(Sk)) > 0.4
+    for mask in (None, kv):
+        _attn_check(gpu, dtype, B, H, Sq, Sk, hd, False, seed=hd + Sk, key_valid=mask)
+        if Sq == Sk:
+            _attn_check(gpu, dtype, B, H, Sq, Sk, hd, True, seed=hd + Sk + 7, key_valid=mask,
+                        packed=True)
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("hd", [8, 48, 256])
+def test_attention_tiled_nonfinite_rows_stay_in_their_queries(gpu, hd, bad):
+    """A non-finite element of one query row, or of a masked-out key's K row, reaches no other row
+    (V rows are always multiplied, by 0 for a masked key, as in the reference)."""
+    ops = _ops()
+    q, k, v = (_rand((1, 70, 2, hd), torch.float16, s).to(gpu) for s in (1, 2, 3))
+    kv = torch.ones(1, 70, dtype=torch.bool, device=gpu)
+    kv[0, 66] = False
+    ref = ops.attention(q, k, v, key_valid=kv)
+    q2, k2 = q.clone(), k.clone()
+    q2[0, 5, 0, 1] = bad
+    k2[0, 66, :, 0] = bad
+    out = ops.attention(q2, k2, v, key_valid=kv)
+    keep = torch.ones(70, dtype=torch.bool, device=gpu)
+    keep[5] = False
+    assert torch.equal(out[:, keep], ref[:, keep])
+    assert torch.equal(out[:, 5, 1], ref[:, 5, 1])
+
+
 # --------------------------------------------------------------- K that fills no whole step
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M,N", [(4100, 4360), (1100, 3000), (600, 1100)])

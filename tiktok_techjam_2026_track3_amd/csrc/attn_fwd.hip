@@ -26,42 +26,9 @@
 //     rest of its sweep, with bit-identical results; non-causal unmasked waves whose bound keeps
 //     every score within +-8 from the start keep mu = 0 (the max-free sweep: branch-free stages).
 // fp32 kernel: one query per lane on VALU (the fp32 configuration is launch-latency bound).
-#include "common.h"
+#include "attn.h"
 
 namespace {
-
-struct AttnArgs {
-  const void* q;
-  const void* k;
-  const void* v;
-  void* o;
-  int64_t qs0, qs1, qs2;  // batch, seq, head strides in elements (head_dim stride 1)
-  int64_t ks0, ks1, ks2;
-  int64_t vs0, vs1, vs2;
-  int64_t os0, os1, os2;
-  int64_t B, H, Sq, Sk;
-  float c;    // scale * log2(e)
-  // key mask [B, S_k] (nullable): applied by the key-masked instances; given to the unmasked
-  // instance together with bounds and redo flags, it only hands work-groups with an invalid key
-  // to the key-masked redo launch
-  const uint8_t* kv;
-  int64_t kv_sb;
-  int n_qtiles;
-  int o_vec;  // output base and strides keep every output row 16-byte aligned
-  // key-norm bounds (nullable; MFMA kernel): kb[(b * H + h) * kb_n + i] = max |k| over key chunk
-  // i of head (b, h), written by attn_key_bound (sign bit set: the chunk holds an invalid key)
-  const float* kb;
-  int kb_n;
-  // causal work-groups take the max-free / offset sweeps only when their key range [0, end of
-  // query tile) holds at least this many keys
-  int64_t sweep_min_k;
-  // redo flags (nullable; MFMA launches without a key mask, or with one and bounds): one int per
-  // work-group (linear block index). The first launch writes every flag: 1 when a row of the
-  // work-group's offset sweep failed its check, or when the work-group visits an invalid key;
-  // the redo launch (the kernel's REDO instance; key-masked when the call has a mask) runs only
-  // the flagged work-groups, without the offset sweep.
-  int* redo;
-};
 
 // Keys per chunk of the key-norm bound pass: the queries of one MFMA work-group, so that a causal
 // work-group reduces the bounds of exactly the keys it visits, [0, end of its query tile) (no
@@ -113,50 +80,6 @@ constexpr bool MAXFREE_INSTANCE = !PIPE && !(CAUSAL && KMASK) && MI355_ATTN_MAXF
 // to spare for it)
 template <bool PIPE, bool CAUSAL, bool KMASK>
 constexpr bool OFFSET_INSTANCE = MAXFREE_INSTANCE<PIPE, CAUSAL, KMASK> && !KMASK;
-
-constexpr float NEG_INF = -__builtin_huge_valf();
-
-// Work-group -> (query tile, head, batch).
-// Non-causal grids are 1-D and XCD-aware: the dispatcher deals work-groups round-robin to the 8
-// XCDs (work-group w runs on XCD w % 8), so XCD x is given the contiguous logical range x*q ..
-// of (head, query tile) pairs, query tile fastest. The query tiles of one head then run on one
-// XCD and share its K/V through that XCD's L2 (dealt round-robin, every XCD would fetch every
-// head's K/V from the fabric). Launches too large for a 1-D dispatch use a (q tiles, H, B) grid.
-// Causal grids are 1-D and issued longest-first over the whole launch: every (batch, head)'s last
-// query tile, then every second-to-last one, ... (a query tile's work grows with its index), so
-// no long tile is left for the end. Consecutive work-groups are different heads; those of one
-// head are H*B apart (on one XCD when H*B is a multiple of 8).
-template <bool CAUSAL>
-MI355_DEVINL void tile_of_block(const AttnArgs& p, int& qt, int64_t& h, int64_t& b) {
-  if constexpr (CAUSAL) {
-    const int64_t lin = blockIdx.x, hb_n = p.H * p.B;
-    qt = p.n_qtiles - 1 - static_cast<int>(lin / hb_n);
-    const int64_t hb = lin % hb_n;
-    h = hb % p.H;
-    b = hb / p.H;
-  } else if (gridDim.y == 1 && gridDim.z == 1) {
-    const int64_t total = gridDim.x;
-    const int64_t q = total / 8, r = total % 8;
-    const int64_t x = blockIdx.x % 8, j = blockIdx.x / 8;
-    const int64_t logical = x * q + (x < r ? x : r) + j;
-    qt = static_cast<int>(logical % p.n_qtiles);
-    const int64_t hb = logical / p.n_qtiles;
-    h = hb % p.H;
-    b = hb / p.H;
-  } else {
-    qt = static_cast<int>(blockIdx.x);
-    h = blockIdx.y;
-    b = blockIdx.z;
-  }
-}
-
-MI355_DEVINL float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
-// IEEE maximum (NaN-propagating): gfx950 v_maximum3_f32, no operand canonicalisation needed
-MI355_DEVINL float vmax(float a, float b) { return __builtin_elementwise_maximum(a, b); }
-MI355_DEVINL float pair_maximum(float v) {
-  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return vmax(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
 
 // XOR swizzle of the 16-byte chunks of K/V LDS rows (NCH chunks per row, row = key). It maps
 // row bits 0..3 onto chunk bits so that both read patterns are free of bank conflicts (checked
@@ -1245,7 +1168,7 @@ __global__ __launch_bounds__(256) void attn_key_bound(AttnArgs p, float* __restr
   }
 }
 
-// VALU kernel: every fp32 problem, and 16-bit head dims the MFMA kernel does not take. LQ lanes
+// VALU kernel: every fp32 problem, and 16-bit ones of a few wide rows (attn_fwd_impl). LQ lanes
 // per query (4, or 2 when head_dim is not a multiple of 16) and 64 / LQ queries per work-group of
 // NWK waves, so the small problems (128 queries x 4 heads) still spread over many CUs. Lane
 // LQ*qq + ds holds the 4-element pieces LQ*j + ds (j < NJ) of query qq's row and of its output
@@ -1643,24 +1566,24 @@ int launch_valu(const AttnArgs& a, bool causal, bool kmask, hipStream_t s) {
   return launch_valu_nwk<T, HD, 8>(a, causal, kmask, s);
 }
 
-// head dims of the VALU kernel (fp32: all of them; 16-bit: all but 64 and 128, which the MFMA
-// kernel takes)
+// head dims of the VALU kernel: fp32 all of them, 16-bit the two that prefer it for a handful of
+// keys (see attn_fwd_impl)
 template <typename T>
 int dispatch_valu(const AttnArgs& a, int64_t hd, bool causal, bool kmask, hipStream_t s) {
-  switch (hd) {
-    case 8: return launch_valu<T, 8>(a, causal, kmask, s);
-    case 16: return launch_valu<T, 16>(a, causal, kmask, s);
-    case 32: return launch_valu<T, 32>(a, causal, kmask, s);
-    case 48: return launch_valu<T, 48>(a, causal, kmask, s);
-    case 80: return launch_valu<T, 80>(a, causal, kmask, s);
-    case 96: return launch_valu<T, 96>(a, causal, kmask, s);
-    case 192: return launch_valu<T, 192>(a, causal, kmask, s);
-    case 256: return launch_valu<T, 256>(a, causal, kmask, s);
-    default: break;
-  }
+  if (hd == 192) return launch_valu<T, 192>(a, causal, kmask, s);
+  if (hd == 256) return launch_valu<T, 256>(a, causal, kmask, s);
   if constexpr (sizeof(T) == 4) {
-    if (hd == 64) return launch_valu<T, 64>(a, causal, kmask, s);
-    if (hd == 128) return launch_valu<T, 128>(a, causal, kmask, s);
+    switch (hd) {
+      case 8: return launch_valu<T, 8>(a, causal, kmask, s);
+      case 16: return launch_valu<T, 16>(a, causal, kmask, s);
+      case 32: return launch_valu<T, 32>(a, causal, kmask, s);
+      case 48: return launch_valu<T, 48>(a, causal, kmask, s);
+      case 64: return launch_valu<T, 64>(a, causal, kmask, s);
+      case 80: return launch_valu<T, 80>(a, causal, kmask, s);
+      case 96: return launch_valu<T, 96>(a, causal, kmask, s);
+      case 128: return launch_valu<T, 128>(a, causal, kmask, s);
+      default: break;
+    }
   }
   return MI355_E_HEAD_DIM;
 }
@@ -1759,8 +1682,13 @@ int attn_fwd_impl(int dtype, const void* Q, const void* K, const void* V, void* 
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype == MI355_F32) return dispatch_valu<float>(a, head_dim, cz, kmask, s);
   if (!on_mfma_kernel(dtype, head_dim)) {
-    return dtype == MI355_F16 ? dispatch_valu<_Float16>(a, head_dim, cz, kmask, s)
-                              : dispatch_valu<__bf16>(a, head_dim, cz, kmask, s);
+    // head dims 192 and 256 over at most 8 queries and keys: a 32-key tile is mostly padding there,
+    // and the vector-ALU kernel, which reads the real rows only, is faster (8192 heads of 4: 32
+    // against 43 us at 256; of 16: 103 against 60)
+    if (head_dim >= 192 && S_q <= 8 && S_k <= 8)
+      return dtype == MI355_F16 ? dispatch_valu<_Float16>(a, head_dim, cz, kmask, s)
+                                : dispatch_valu<__bf16>(a, head_dim, cz, kmask, s);
+    return mi355_internal_attn_tiled({&a, head_dim, dtype == MI355_BF16, cz}, s);
   }
   float* kb = nullptr;
   int* redo = nullptr;
