@@ -871,6 +871,23 @@ def test_attention_tiled_nonfinite_rows_stay_in_their_queries(gpu, hd, bad):
     assert torch.equal(out[:, 5, 1], ref[:, 5, 1])
 
 
+# ------------------------------------------------------------- fp32 attention on fp32 MFMAs
+@pytest.mark.parametrize("hd", [8, 16, 32, 48, 64, 80, 96, 128, 192, 256])
+@pytest.mark.parametrize("B,Sq,Sk", [(260, 64, 64), (260, 64, 1), (130, 65, 97), (130, 128, 130),
+                                     (66, 129, 129), (33, 257, 40)])
+def test_attention_f32_mfma_edges(gpu, hd, B, Sq, Sk):
+    """Enough (batch, head, query tile) work-groups for attn_fwd_f32, at the edges of its query and
+    key tiles, with and without a key mask; packed views and causal where S_q = S_k."""
+    B = B if hd <= 64 else B // 2
+    kv = torch.ones(B, Sk, dtype=torch.bool)
+    kv[:, (Sk + 1) // 2:] = torch.rand(B, Sk // 2, generator=torch.Generator().manual_seed(Sk)) > 0.4
+    for mask in (None, kv):
+        _attn_check(gpu, torch.float32, B, 2, Sq, Sk, hd, False, seed=hd + Sk, key_valid=mask)
+        if Sq == Sk:
+            _attn_check(gpu, torch.float32, B, 2, Sq, Sk, hd, True, seed=hd + 7, key_valid=mask,
+                        packed=True)
+
+
 # --------------------------------------------------------------- K that fills no whole step
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M,N", [(4100, 4360), (1100, 3000), (600, 1100)])

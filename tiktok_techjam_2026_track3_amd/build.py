@@ -50,7 +50,7 @@ def sources() -> list[Path]:
 # them with hand-placed s_waitcnt / barriers. They must not use scratch memory: spill stores and
 # reloads are vector-memory operations the hand-placed counts do not account for, and a spilling
 # build of the attention loader produced nondeterministic rows. The build refuses such a kernel.
-NO_SCRATCH_KERNELS = re.compile(r"attn_fwd_mfma|attn_fwd_tiled|gemm_kernel")
+NO_SCRATCH_KERNELS = re.compile(r"attn_fwd_mfma|attn_fwd_tiled|attn_fwd_f32|gemm_kernel")
 _REMARK = re.compile(r"remark:\s+(Function Name|ScratchSize \[bytes/lane\]|VGPRs Spill|SGPRs Spill):\s+(\S+)")
 
 

@@ -93,3 +93,8 @@ struct AttnTiledCall {
 };
 __attribute__((visibility("hidden"))) int mi355_internal_attn_tiled(const AttnTiledCall& call,
                                                                     hipStream_t s);
+// attn_f32.hip: fp32 attention on fp32 MFMAs, every head dim, and whether it is the faster kernel
+// for the problem (against the vector-ALU one).
+__attribute__((visibility("hidden"))) bool mi355_internal_attn_f32_wins(const AttnTiledCall& call);
+__attribute__((visibility("hidden"))) int mi355_internal_attn_f32(const AttnTiledCall& call,
+                                                                  hipStream_t s);

@@ -1168,7 +1168,7 @@ __global__ __launch_bounds__(256) void attn_key_bound(AttnArgs p, float* __restr
   }
 }
 
-// VALU kernel: every fp32 problem, and 16-bit ones of a few wide rows (attn_fwd_impl). LQ lanes
+// VALU kernel: fp32 problems of few query tiles, 16-bit ones of a few wide rows (attn_fwd_impl). LQ lanes
 // per query (4, or 2 when head_dim is not a multiple of 16) and 64 / LQ queries per work-group of
 // NWK waves, so the small problems (128 queries x 4 heads) still spread over many CUs. Lane
 // LQ*qq + ds holds the 4-element pieces LQ*j + ds (j < NJ) of query qq's row and of its output
@@ -1680,7 +1680,11 @@ int attn_fwd_impl(int dtype, const void* Q, const void* K, const void* V, void* 
   const bool kmask = key_valid != nullptr;
   const bool cz = causal != 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (dtype == MI355_F32) return dispatch_valu<float>(a, head_dim, cz, kmask, s);
+  if (dtype == MI355_F32) {
+    const AttnTiledCall call = {&a, head_dim, false, cz};
+    if (mi355_internal_attn_f32_wins(call)) return mi355_internal_attn_f32(call, s);
+    return dispatch_valu<float>(a, head_dim, cz, kmask, s);
+  }
   if (!on_mfma_kernel(dtype, head_dim)) {
     // head dims 192 and 256 over at most 8 queries and keys: a 32-key tile is mostly padding there,
     // and the vector-ALU kernel, which reads the real rows only, is faster (8192 heads of 4: 32
