@@ -355,6 +355,24 @@ int mi355_layernorm_gemm_bias_noalloc(int in_dtype, int out_dtype, const void* X
                                       const float* bias, float eps, void* C, int64_t ldc, int64_t M,
                                       int64_t N, int64_t K, int epi, void* stream);
 
+/*
+ * The rest of a narrow transformer block after its attention, in one launch
+ * (torch_transformer_benchmark.py:118-121, :139-145):
+ *     x1 = X + (ctx W_o^T + b_o), masked rows X;   Y = x1 + gelu(norm2(x1) W_in^T + b_in) W_out^T + b_out,
+ * masked rows 0, with the rounding points of mi355_gemm_bias_residual, mi355_layernorm(_cvt) to
+ * fp16, mi355_gemm_bias_gelu (fp16 output) and mi355_gemm_bias_residual_zero_masked. dtype is X's,
+ * Y's, gamma's and beta's (F32 or F16); ctx and the contiguous weights W_o [d, d], W_in [ffn, d],
+ * W_out [d, ffn] are fp16, the biases fp32; biases, gamma, beta and row_valid may be NULL. Y may be
+ * X. ctx, the weights and the biases are 16-byte aligned, X, Y, gamma and beta to four elements;
+ * ldc is a multiple of 8, ldx and ldy of 4. (d_model, ffn_dim) other than (32, 32 | 64 | 128),
+ * (64, 64 | 128) and (128, 64 | 128) return MI355_E_UNSUPPORTED, nothing launched: run those calls.
+ */
+int mi355_block_tail(int dtype, const void* ctx, int64_t ldc, const void* X, int64_t ldx, void* Y,
+                     int64_t ldy, const void* W_o, const float* b_o, const void* gamma,
+                     const void* beta, float eps, const void* W_in, const float* b_in,
+                     const void* W_out, const float* b_out, int64_t M, int64_t d_model,
+                     int64_t ffn_dim, const uint8_t* row_valid, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -530,3 +530,81 @@ def test_int8_plugin_full_model_equals_transformer(gpu, dtype):
                                                                           mask, True))
         out = fused(x, mask)
     assert torch.isfinite(out).all() and torch.all(out[~mask] == 0)
+
+
+# ------------------------------------------------------------- the narrow block's fused tail
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("d,ffn", [(32, 32), (32, 128), (64, 64), (64, 128), (128, 64), (128, 128)])
+@pytest.mark.parametrize("M", [1, 63, 65, 1000, 65536 + 131])
+def test_block_tail(gpu, dtype, d, ffn, M):
+    """ops.block_tail against the four launches it stands for, at the edges of its row tiles (64
+    rows, persistent from 256 per CU on): the same residual stream (W_out = 0; bit for bit where
+    the out projection is the tiled GEMM, whose products run in the same order), and no larger error against fp64 than theirs (the LayerNorm sums run in another order, so a
+    normalised element next to a rounding boundary may differ by an fp16 step)."""
+    from tiktok_techjam_2026_track3_amd import ops
+    g = torch.Generator(device=gpu).manual_seed(d + ffn + M)
+
+    def r(*s, scale=1.0):
+        return torch.randn(*s, generator=g, device=gpu) * scale
+
+    ctx, x = r(M, d).half(), (r(M, d) * 2 + 0.5).to(dtype)
+    w_o, w_in, w_out = (r(d, d, scale=d ** -0.5).half(), r(ffn, d, scale=d ** -0.5).half(),
+                        r(d, ffn, scale=ffn ** -0.5).half())
+    b_o, b_in, b_out = r(d), r(ffn), r(d)
+    gm, bt = (r(d) * 0.3 + 1).to(dtype), (r(d) * 0.2).to(dtype)
+    rv = r(M) > -0.5
+    rv[0] = True
+    print(f"block tail {dtype} d={d} ffn={ffn} M={M}", flush=True)
+
+    def separate(wt, bb, mask):
+        x1 = ops.linear(ctx, w_o, b_o, row_valid=mask, residual=x, out_dtype=dtype)
+        h = ops.layer_norm(x1, gm, bt, 1e-5, out_dtype=torch.float16)
+        gg = ops.linear(h, w_in, b_in, gelu=True, out_dtype=torch.float16)
+        return x1, ops.linear(gg, wt, bb, residual=x1, row_valid=mask, zero_masked_rows=True,
+                              out_dtype=dtype)
+
+    for mask in (None, rv):
+        zero = torch.zeros_like(w_out)
+        x1, y0 = separate(zero, None, mask)
+        z0 = ops.block_tail(ctx, x, w_o, b_o, gm, bt, 1e-5, w_in, b_in, zero, None, row_valid=mask)
+        if M > 60000:
+            assert torch.equal(z0, y0)
+        else:
+            # the split-K kernel sums in another order: each side within K 2^-24 sum|ctx w| of the
+            # exact projection, and (fp16) one rounding step of it and of the sum apart
+            mag = ctx.double().abs() @ w_o.double().abs().T + b_o.double().abs() + x.double().abs()
+            tol = 2 * d * 2.0 ** -24 * mag
+            if dtype == torch.float16:
+                tol = tol + 2 * 2.0 ** -10 * mag
+            assert torch.all((z0.double() - y0.double()).abs() <= tol)
+        sep = separate(w_out, b_out, mask)[1]
+        got = ops.block_tail(ctx, x, w_o, b_o, gm, bt, 1e-5, w_in, b_in, w_out, b_out,
+                             row_valid=mask)
+        x64 = ctx.double() @ w_o.double().T + b_o.double()
+        x64 = x.double() + (x64 if mask is None else x64 * mask[:, None])
+        n = (x64 - x64.mean(1, keepdim=True)) / torch.sqrt(
+            x64.var(1, unbiased=False, keepdim=True) + 1e-5) * gm.double() + bt.double()
+        f = n @ w_in.double().T + b_in.double()
+        f = 0.5 * f * (1 + torch.erf(f * 2 ** -0.5))
+        ref = x64 + f @ w_out.double().T + b_out.double()
+        if mask is not None:
+            ref = ref * mask[:, None]
+            assert torch.all(got[~mask] == 0)
+        e_sep, e_got = ((t.double() - ref).norm() / ref.norm() for t in (sep, got))
+        worst = float((got.double() - sep.double()).abs().max() / sep.double().abs().max())
+        print(f"  error {float(e_got):.3g}, separate {float(e_sep):.3g}, apart {worst:.3g}", flush=True)
+        assert e_got <= 1.05 * e_sep + 1e-7
+        # a few fp16 steps of h and g, each times |w| ~ 1 / sqrt(k), over the row
+        assert worst <= 8 * 2.0 ** -11
+
+
+def test_block_tail_unsupported_size_and_nulls(gpu):
+    from tiktok_techjam_2026_track3_amd import ops
+    from tiktok_techjam_2026_track3_amd._lib import KernelError
+    z = lambda *s: torch.zeros(*s, dtype=torch.float16, device=gpu)  # noqa: E731
+    with pytest.raises(KernelError):
+        ops.block_tail(z(4, 96), z(4, 96), z(96, 96), None, None, None, 1e-5, z(96, 96), None,
+                       z(96, 96), None)
+    out = ops.block_tail(z(4, 64), z(4, 64), z(64, 64), None, None, None, 1e-5, z(64, 64), None,
+                         z(64, 64), None)
+    assert torch.all(out == 0)

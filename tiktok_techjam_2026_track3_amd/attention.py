@@ -333,6 +333,17 @@ class SelfAttention(nn.Module):
         extra "norm" stage before "qkv".
         """
         mark = marks or (lambda _stage: None)
+        ctx, x2, row_valid, w_o, b_o = self._normed_context(x, norm, valid_token_mask, causal, mark)
+        mark("out")
+        out = ops.linear(ctx, w_o, b_o, row_valid=row_valid, out_dtype=x.dtype, residual=x2)
+        mark("end")
+        return out.view(x.shape)
+
+    def _normed_context(self, x: torch.Tensor, norm: nn.LayerNorm,
+                        valid_token_mask: Optional[torch.Tensor], causal: bool,
+                        mark: Callable[[str], None]):
+        """norm, QKV projection and attention of ``forward_residual``: ``(ctx [T, d], x [T, d],
+        row_valid, W_o, b_o)``, what the out projection and the residual need."""
         B, S = self._check_input(x)
         d = self.d_model
         if tuple(norm.normalized_shape) != (d,):
@@ -363,11 +374,7 @@ class SelfAttention(nn.Module):
         q, k, v = self._qkv_views(qkv, B, S)
         mark("attn")
         ctx = self._attend(q, k, v, causal, key_valid, kbt)
-        mark("out")
-        out = ops.linear(ctx.view(B * S, d), w_o, b_o, row_valid=row_valid, out_dtype=x.dtype,
-                         residual=x2)
-        mark("end")
-        return out.view(B, S, d)
+        return ctx.view(B * S, d), x2, row_valid, w_o, b_o
 
 
 class Int8SelfAttention(SelfAttention):

@@ -1,0 +1,295 @@
+// The row-local rest of a narrow transformer block after its attention, in one kernel:
+//   x1 = x + out_proj(ctx)                       (masked rows: x)
+//   y  = x1 + ffn_out(gelu(ffn_in(norm2(x1))))   (masked rows: 0)
+// with fp16 operands, for blocks whose three weight matrices fit the LDS together (d_model and
+// ffn_dim up to 128). The four launches it replaces (out projection + residual, LayerNorm, ffn_in +
+// GELU, ffn_out + residual) are bound by their passes over memory there: per row of 128 fp32
+// features 256 + 512 + 512, 512 + 256, 256 + 256 and 256 + 512 + 512 bytes, here 256 + 512 + 512.
+//
+// A wave owns RT blocks of 16 rows from the context to the output and nothing crosses waves. Each
+// product is formed transposed on 16x16x32 MFMAs (A = 16 weight rows from LDS, B = 16 rows of the
+// activations), which leaves lane l four consecutive features 4 (l / 16) .. of row l % 16 per
+// block. That is the residual's and the output's layout (16-byte accesses), a row's sums are one
+// exchange over four lanes, and two blocks of it are the next product's B operand once that weight
+// is stored with its k order permuted to match (stage_weight): x1, the normalised row and the GELU
+// output stay in registers. The rounding points are those of the separate launches. [1280000, 128]
+// fp32: the four launches 1425 us, this one 430; the official 4-layer model over 10 000 sequences
+// 10.42 -> 5.49 ms, over 64 0.210 -> 0.162.
+#include <type_traits>
+
+#include "common.h"
+
+namespace {
+
+struct TailArgs {
+  const _Float16* ctx;  // [M, D], row stride ldc
+  const void* x;        // [M, D] residual stream, row stride ldx
+  void* y;              // [M, D], row stride ldy; may be x
+  const _Float16 *wo, *w1, *w2;  // [D, D], [F, D], [D, F], contiguous
+  const float *bo, *b1, *b2;     // nullable
+  const void *gamma, *beta;      // [D] of x's type, nullable
+  const uint8_t* row_valid;      // nullable
+  int64_t ldc, ldx, ldy, M;
+  float eps;
+};
+
+// XOR of the 16-byte chunks of a weight's LDS row (NCH of them): conflict-free fragment reads (lane
+// l's row l % 16, chunk c + l / 16)
+template <int NCH>
+MI355_DEVINL int swz_w(int r) {
+  if constexpr (NCH % 16 == 0)
+    return r & 15;
+  else if constexpr (NCH == 8)
+    return (r >> 1) & 7;
+  else
+    return (4 - (r >> 2)) & 3;
+}
+
+// W [N, K] into LDS, rows of K / 8 swizzled chunks. PERM: chunk q of a 32-wide k-step holds k
+// 4 q .. + 3 and 16 + 4 q .. + 3 of it instead of 8 q .. + 7 (see the head of the file).
+template <int N, int K, int NT, bool PERM>
+MI355_DEVINL void stage_weight(u32x4* lds, const _Float16* __restrict__ w) {
+  constexpr int NCH = K / 8;
+  for (int i = threadIdx.x; i < N * NCH; i += NT) {
+    const int r = i / NCH, c = i % NCH;
+    u32x4 v;
+    if constexpr (PERM) {
+      const _Float16* src = w + r * K + c / 4 * 32 + c % 4 * 4;
+      const u32x2 lo = *reinterpret_cast<const u32x2*>(src), hi = *reinterpret_cast<const u32x2*>(src + 16);
+      v = u32x4{lo[0], lo[1], hi[0], hi[1]};
+    } else {
+      v = *reinterpret_cast<const u32x4*>(w + r * K + c * 8);
+    }
+    lds[r * NCH + (c ^ swz_w<NCH>(r))] = v;
+  }
+}
+
+MI355_DEVINL float quad_add(float v) {  // over lanes l, l ^ 16, l ^ 32, l ^ 48
+  v = pair_sum(v);
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+template <typename T>
+MI355_DEVINL f32x4 load4f(const T* p) {
+  if constexpr (sizeof(T) == 4) {
+    return *reinterpret_cast<const f32x4*>(p);
+  } else {
+    const f16x4 v = *reinterpret_cast<const f16x4*>(p);
+    return f32x4{to_f32(v[0]), to_f32(v[1]), to_f32(v[2]), to_f32(v[3])};
+  }
+}
+
+template <typename T, int D, int F, int NW, int RT>
+__global__ __launch_bounds__(NW * 64, NW / 4) void block_tail(TailArgs p) {
+  static_assert(D % 32 == 0 && F % 32 == 0, "whole MFMA steps");
+  constexpr int DB = D / 16, FB = F / 16, NT = NW * 64, ROWS = 16 * RT * NW;
+  __shared__ u32x4 lds_o[D * D / 8], lds_1[F * D / 8], lds_2[D * F / 8];
+  stage_weight<D, D, NT, false>(lds_o, p.wo);
+  stage_weight<F, D, NT, true>(lds_1, p.w1);
+  stage_weight<D, F, NT, true>(lds_2, p.w2);
+  __syncthreads();
+
+  const int lane = threadIdx.x & 63, q = lane >> 4, l16 = lane & 15;
+  const int wave = threadIdx.x >> 6;
+  // Keeps a k-step's weight fragments where they are used: the compiler would otherwise hoist the
+  // reads of all three matrices (they do not change) into registers, out of the row loop even.
+  auto fence = [] {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // acc[r][fb] = W[16 fb .., :] . B[r]^T
+  auto product = [&](auto nb_c, auto k_c, const u32x4* w, auto& frag, auto& acc) MI355_LAMBDA_INLINE {
+    constexpr int NB = decltype(nb_c)::value, K = decltype(k_c)::value, NCH = K / 8;
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int fb = 0; fb < NB; ++fb) acc[r][fb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < K / 32; ++s) {
+      fence();
+#pragma unroll
+      for (int fb = 0; fb < NB; ++fb) {
+        const int row = 16 * fb + l16, c = 4 * s + q;
+        const f16x8 wf = __builtin_bit_cast(f16x8, w[row * NCH + (c ^ swz_w<NCH>(row))]);
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+          acc[r][fb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf, frag[r][s], acc[r][fb], 0, 0, 0);
+      }
+    }
+    fence();
+  };
+  // features 16 fb + 4 q .. + 3 of a bias
+  auto bias4 = [&](const float* b, int fb) MI355_LAMBDA_INLINE {
+    return b != nullptr ? *reinterpret_cast<const f32x4*>(b + 16 * fb + 4 * q) : f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  using cD = std::integral_constant<int, D>;
+  using cF = std::integral_constant<int, F>;
+  using cDB = std::integral_constant<int, DB>;
+  using cFB = std::integral_constant<int, FB>;
+
+  for (int64_t base = static_cast<int64_t>(blockIdx.x) * ROWS; base < p.M; base += static_cast<int64_t>(gridDim.x) * ROWS) {
+    int64_t row[RT];
+    bool in[RT], valid[RT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      row[r] = base + (wave * RT + r) * 16 + l16;
+      in[r] = row[r] < p.M;
+      if (!in[r]) row[r] = p.M - 1;  // a real row, computed again and not stored
+      valid[r] = p.row_valid == nullptr || p.row_valid[row[r]] != 0;
+    }
+    f16x8 cf[RT][D / 32];
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int s = 0; s < D / 32; ++s)
+        cf[r][s] = *reinterpret_cast<const f16x8*>(p.ctx + row[r] * p.ldc + 32 * s + 8 * q);
+    f32x4 x1[RT][DB];
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int fb = 0; fb < DB; ++fb)
+        x1[r][fb] = load4f(static_cast<const T*>(p.x) + row[r] * p.ldx + 16 * fb + 4 * q);
+
+    // x1 = x + out_proj(ctx): the projection rounded to x's type, masked rows 0, then the sum
+    f32x4 acc[RT][DB];
+    product(cDB{}, cD{}, lds_o, cf, acc);
+#pragma unroll
+    for (int fb = 0; fb < DB; ++fb) {
+      fence();
+      const f32x4 b = bias4(p.bo, fb);
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float v = valid[r] ? acc[r][fb][e] + b[e] : 0.f;
+          x1[r][fb][e] = to_f32(from_f32<T>(to_f32(from_f32<T>(v)) + x1[r][fb][e]));
+        }
+    }
+    fence();
+    // norm2, as the LayerNorm kernel: mean and biased variance by two passes over the registers
+    f16x8 h[RT][D / 32];
+    float mean[RT], rstd[RT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      float sum = 0.f;
+#pragma unroll
+      for (int fb = 0; fb < DB; ++fb) sum += (x1[r][fb][0] + x1[r][fb][1]) + (x1[r][fb][2] + x1[r][fb][3]);
+      mean[r] = quad_add(sum) / static_cast<float>(D);
+      float sq = 0.f;
+#pragma unroll
+      for (int fb = 0; fb < DB; ++fb)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float d = x1[r][fb][e] - mean[r];
+          sq += d * d;
+        }
+      rstd[r] = 1.0f / sqrtf(quad_add(sq) / static_cast<float>(D) + p.eps);
+    }
+#pragma unroll
+    for (int fb = 0; fb < DB; ++fb) {
+      fence();
+      f32x4 gm = {1.f, 1.f, 1.f, 1.f}, bt = {0.f, 0.f, 0.f, 0.f};
+      if (p.gamma) gm = load4f(static_cast<const T*>(p.gamma) + 16 * fb + 4 * q);
+      if (p.beta) bt = load4f(static_cast<const T*>(p.beta) + 16 * fb + 4 * q);
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          h[r][fb / 2][4 * (fb % 2) + e] = from_f32<_Float16>((x1[r][fb][e] - mean[r]) * rstd[r] * gm[e] + bt[e]);
+    }
+    // g = gelu(ffn_in(h)): the projection rounded to fp16, then its GELU
+    f16x8 g[RT][F / 32];
+    {
+      f32x4 a1[RT][FB];
+      product(cFB{}, cD{}, lds_1, h, a1);
+#pragma unroll
+      for (int fb = 0; fb < FB; ++fb) {
+        fence();
+        const f32x4 b = bias4(p.b1, fb);
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            g[r][fb / 2][4 * (fb % 2) + e] =
+                from_f32<_Float16>(gelu_erf(to_f32(from_f32<_Float16>(a1[r][fb][e] + b[e]))));
+      }
+    }
+    // y = x1 + ffn_out(g), masked rows 0
+    product(cDB{}, cF{}, lds_2, g, acc);
+#pragma unroll
+    for (int fb = 0; fb < DB; ++fb) {
+      fence();
+      const f32x4 b = bias4(p.b2, fb);
+#pragma unroll
+      for (int r = 0; r < RT; ++r) {
+        typedef T t4 __attribute__((ext_vector_type(4)));
+        t4 w;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float v = to_f32(from_f32<T>(acc[r][fb][e] + b[e])) + x1[r][fb][e];
+          w[e] = from_f32<T>(valid[r] ? v : 0.f);
+        }
+        if (in[r]) *reinterpret_cast<t4*>(static_cast<T*>(p.y) + row[r] * p.ldy + 16 * fb + 4 * q) = w;
+      }
+    }
+  }
+}
+
+// Persistent work-groups of 8 waves of two row blocks, which stage the weights once; 4 waves of one
+// where that would leave CUs without rows.
+template <typename T, int D, int F>
+int launch(const TailArgs& a, hipStream_t s) {
+  constexpr int64_t BIG = 16 * 2 * 8, SMALL = 16 * 4;
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    return static_cast<int>(hipGetLastError());
+  if (a.M >= BIG * cus) {
+    hipLaunchKernelGGL((block_tail<T, D, F, 8, 2>), dim3(static_cast<unsigned>(cus)), dim3(512), 0, s, a);
+  } else {
+    const int64_t n = (a.M + SMALL - 1) / SMALL;
+    hipLaunchKernelGGL((block_tail<T, D, F, 4, 1>), dim3(static_cast<unsigned>(n)), dim3(256), 0, s, a);
+  }
+  return static_cast<int>(hipGetLastError());
+}
+
+template <typename T>
+int dispatch(const TailArgs& a, int64_t d, int64_t f, hipStream_t s) {
+  if (d == 32 && f == 32) return launch<T, 32, 32>(a, s);
+  if (d == 32 && f == 64) return launch<T, 32, 64>(a, s);
+  if (d == 32 && f == 128) return launch<T, 32, 128>(a, s);
+  if (d == 64 && f == 64) return launch<T, 64, 64>(a, s);
+  if (d == 64 && f == 128) return launch<T, 64, 128>(a, s);
+  if (d == 128 && f == 64) return launch<T, 128, 64>(a, s);
+  if (d == 128 && f == 128) return launch<T, 128, 128>(a, s);
+  return MI355_E_UNSUPPORTED;
+}
+
+}  // namespace
+
+extern "C" int mi355_block_tail(int dtype, const void* ctx, int64_t ldc, const void* X, int64_t ldx,
+                                void* Y, int64_t ldy, const void* W_o, const float* b_o,
+                                const void* gamma, const void* beta, float eps, const void* W_in,
+                                const float* b_in, const void* W_out, const float* b_out, int64_t M,
+                                int64_t d_model, int64_t ffn_dim, const uint8_t* row_valid,
+                                void* stream) {
+  if (M < 0 || d_model <= 0 || ffn_dim <= 0) return MI355_E_BAD_SIZE;
+  if (dtype != MI355_F32 && dtype != MI355_F16) return MI355_E_BAD_DTYPE;
+  if (M == 0) return MI355_OK;
+  if (!ctx || !X || !Y || !W_o || !W_in || !W_out) return MI355_E_NULL_POINTER;
+  if (!(eps >= 0.f) || ldc < d_model || ldx < d_model || ldy < d_model) return MI355_E_BAD_SIZE;
+  // 16-byte accesses of the context, weights and biases, four elements of the rest
+  const int64_t vx = dtype == MI355_F32 ? 15 : 7;
+  auto off = [](const void* p, int64_t mask) { return (reinterpret_cast<uintptr_t>(p) & mask) != 0; };
+  if (ldc % 8 || ldx % 4 || ldy % 4 || off(ctx, 15) || off(X, vx) || off(Y, vx) || off(W_o, 15) ||
+      off(W_in, 15) || off(W_out, 15) || off(b_o, 15) || off(b_in, 15) || off(b_out, 15) ||
+      off(gamma, vx) || off(beta, vx))
+    return MI355_E_ALIGNMENT;
+  TailArgs a{static_cast<const _Float16*>(ctx), X, Y, static_cast<const _Float16*>(W_o),
+             static_cast<const _Float16*>(W_in), static_cast<const _Float16*>(W_out), b_o, b_in, b_out,
+             gamma, beta, row_valid, ldc, ldx, ldy, M, eps};
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  return dtype == MI355_F32 ? dispatch<float>(a, d_model, ffn_dim, s)
+                            : dispatch<_Float16>(a, d_model, ffn_dim, s);
+}

@@ -40,30 +40,6 @@ MI355_DEVINL float ln_fold(float acc, float mean, float rstd, float colsum, floa
   return __builtin_fmaf(rstd, __builtin_fmaf(-mean, colsum, acc), bias);
 }
 
-// Exact GELU, x * Phi(x) with Phi(x) = erfc(-x / sqrt 2) / 2, in fp32. erfc comes from the
-// Chebyshev fit of Numerical Recipes (Press et al., "erfcc"; fractional error below 1.2e-7 for
-// every argument):  erfc(z) = t exp(-z^2 - 1.26551223 + t P(t)),  t = 1 / (1 + z / 2),  z >= 0,
-// with erfc(-z) = 2 - erfc(z) for the other sign. Branch-free (one reciprocal, one exponential,
-// twelve FMAs): the epilogue evaluates it on every output of a 256 x 256 tile, where a
-// general-purpose erff with range branches cost ~50% of the GEMM's time.
-MI355_DEVINL float gelu_erf(float x) {
-  const float z = __builtin_fabsf(x) * 0.70710678118654752f;
-  const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(0.5f, z, 1.0f));
-  float p = 0.17087277f;
-  p = __builtin_fmaf(p, t, -0.82215223f);
-  p = __builtin_fmaf(p, t, 1.48851587f);
-  p = __builtin_fmaf(p, t, -1.13520398f);
-  p = __builtin_fmaf(p, t, 0.27886807f);
-  p = __builtin_fmaf(p, t, -0.18628806f);
-  p = __builtin_fmaf(p, t, 0.09678418f);
-  p = __builtin_fmaf(p, t, 0.37409196f);
-  p = __builtin_fmaf(p, t, 1.00002368f);
-  const float arg = __builtin_fmaf(t, p, __builtin_fmaf(-z, z, -1.26551223f));
-  const float half_erfc = 0.5f * t * __builtin_amdgcn_exp2f(arg * 1.4426950408889634f);
-  const float phi = x >= 0.f ? 1.0f - half_erfc : half_erfc;
-  return x * phi;
-}
-
 template <typename TO>
 MI355_DEVINL void store_out(void* C, int64_t idx, float v) {
   static_cast<TO*>(C)[idx] = from_f32<TO>(v);

@@ -375,6 +375,52 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: Optional[t
     return out
 
 
+# (d_model, ffn_dim) that block_tail takes: three fp16 weight matrices resident in LDS
+BLOCK_TAIL_SIZES = frozenset(((32, 32), (32, 64), (32, 128), (64, 64), (64, 128), (128, 64),
+                              (128, 128)))
+
+
+def block_tail(ctx: torch.Tensor, x: torch.Tensor, w_o: torch.Tensor, b_o: Optional[torch.Tensor],
+               norm_w: Optional[torch.Tensor], norm_b: Optional[torch.Tensor], eps: float,
+               w_in: torch.Tensor, b_in: Optional[torch.Tensor], w_out: torch.Tensor,
+               b_out: Optional[torch.Tensor],
+               row_valid: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """The row-local rest of a narrow block after its attention, in one launch: ``x1 = x +
+    linear(ctx, w_o, b_o)`` (masked rows x), then ``x1 + linear(gelu(linear(layer_norm(x1), w_in,
+    b_in)), w_out, b_out)`` with masked rows 0, rounded where ``linear`` / ``layer_norm`` with fp16
+    operands round. ``ctx`` ([M, d] fp16, unit column stride) and the weights are fp16, the biases
+    fp32, ``x`` ([M, d]), ``norm_w`` and ``norm_b`` of one type, fp32 or fp16. (d, ffn) must be in
+    ``BLOCK_TAIL_SIZES``."""
+    _on_gpu(ctx, x, w_o, b_o, norm_w, norm_b, w_in, b_in, w_out, b_out, row_valid)
+    if ctx.dim() != 2 or x.dim() != 2 or ctx.shape != x.shape:
+        raise ValueError("block_tail expects 2-D ctx and x of one shape")
+    M, d = x.shape
+    ffn = w_in.shape[0]
+    for t, shape in ((w_o, (d, d)), (w_in, (ffn, d)), (w_out, (d, ffn))):
+        if tuple(t.shape) != shape or t.dtype != torch.float16 or not t.is_contiguous():
+            raise ValueError(f"weights must be contiguous fp16, [{d}, {d}], [ffn, {d}], [{d}, ffn]")
+    if ctx.dtype != torch.float16 or x.dtype not in (torch.float32, torch.float16):
+        raise TypeError("ctx must be fp16 and x fp32 or fp16")
+    if ctx.stride(1) != 1 or x.stride(1) != 1:
+        raise ValueError("ctx and x need unit column stride")
+    for t, n, dt in ((b_o, d, torch.float32), (b_in, ffn, torch.float32), (b_out, d, torch.float32),
+                     (norm_w, d, x.dtype), (norm_b, d, x.dtype)):
+        if t is not None and (tuple(t.shape) != (n,) or t.dtype != dt or not t.is_contiguous()):
+            raise ValueError("biases must be contiguous fp32 and the norm's parameters of x's dtype")
+    y = torch.empty((M, d), device=x.device, dtype=x.dtype)
+
+    def ptr(t):
+        return t.data_ptr() if t is not None else 0
+
+    st = _lib.lib().mi355_block_tail(
+        _lib.dtype_code(x.dtype), ctx.data_ptr(), ctx.stride(0), x.data_ptr(), x.stride(0),
+        y.data_ptr(), y.stride(0), w_o.data_ptr(), ptr(b_o), ptr(norm_w), ptr(norm_b), float(eps),
+        w_in.data_ptr(), ptr(b_in), w_out.data_ptr(), ptr(b_out), M, d, ffn,
+        _mask_ptr(row_valid, (M,)), _stream(x))
+    _lib.check("mi355_block_tail", st)
+    return y
+
+
 def quant_rows_i8(x: torch.Tensor, mode: int = 0) -> Tuple[torch.Tensor, torch.Tensor]:
     """Per-row symmetric int8 quantisation; returns ``(q [M, K] int8, scale [M] fp32)``.
 
