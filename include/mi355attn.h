@@ -373,6 +373,18 @@ int mi355_block_tail(int dtype, const void* ctx, int64_t ldc, const void* X, int
                      const void* W_out, const float* b_out, int64_t M, int64_t d_model,
                      int64_t ffn_dim, const uint8_t* row_valid, void* stream);
 
+/*
+ * norm1 and the packed QKV projection of a narrow block on fp16 operands in one launch:
+ *     Y [M, 3 d] fp16 = fp16(LayerNorm(X)) W_qkv^T + b_qkv
+ * with the rounding points of mi355_layernorm(_cvt) to fp16 followed by mi355_gemm_bias. dtype (F32
+ * or F16) is X's, gamma's and beta's; W_qkv [3 d, d] is fp16 and contiguous, b_qkv fp32; gamma, beta
+ * and b_qkv may be NULL. W_qkv, b_qkv and Y are 16-byte aligned, X, gamma and beta to four elements;
+ * ldx is a multiple of 4, ldy of 8. d_model other than 32, 64 and 128 returns MI355_E_UNSUPPORTED.
+ */
+int mi355_block_head(int dtype, const void* X, int64_t ldx, const void* gamma, const void* beta,
+                     float eps, const void* W_qkv, const float* b_qkv, void* Y, int64_t ldy,
+                     int64_t M, int64_t d_model, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

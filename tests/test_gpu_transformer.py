@@ -608,3 +608,38 @@ def test_block_tail_unsupported_size_and_nulls(gpu):
     out = ops.block_tail(z(4, 64), z(4, 64), z(64, 64), None, None, None, 1e-5, z(64, 64), None,
                          z(64, 64), None)
     assert torch.all(out == 0)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("M", [1, 63, 65, 1000, 65536 + 131])
+def test_block_head(gpu, dtype, d, M):
+    """ops.block_head against LayerNorm kernel + projection at the edges of its row tiles: no larger
+    error against fp64, and apart by a few fp16 steps at most (the LayerNorm sums run in another
+    order); a row of equal elements gives the projection of beta."""
+    from tiktok_techjam_2026_track3_amd import ops
+    g = torch.Generator(device=gpu).manual_seed(d + M)
+
+    def r(*s, scale=1.0):
+        return torch.randn(*s, generator=g, device=gpu) * scale
+
+    x, w, b = (r(M, d) * 2 + 0.5).to(dtype), r(3 * d, d, scale=d ** -0.5).half(), r(3 * d)
+    gm, bt = (r(d) * 0.3 + 1).to(dtype), (r(d) * 0.2).to(dtype)
+    x[-1] = 0.75
+    print(f"block head {dtype} d={d} M={M}", flush=True)
+    h = ops.layer_norm(x, gm, bt, 1e-5, out_dtype=torch.float16)
+    sep, got = ops.linear(h, w, b, out_dtype=torch.float16), ops.block_head(x, gm, bt, 1e-5, w, b)
+    x64 = x.double()
+    n = (x64 - x64.mean(1, keepdim=True)) / torch.sqrt(
+        x64.var(1, unbiased=False, keepdim=True) + 1e-5) * gm.double() + bt.double()
+    ref = n @ w.double().T + b.double()
+    e_sep, e_got = ((t.double() - ref).norm() / ref.norm() for t in (sep, got))
+    worst = float((got.double() - sep.double()).abs().max() / sep.double().abs().max())
+    print(f"  error {float(e_got):.3g}, separate {float(e_sep):.3g}, apart {worst:.3g}", flush=True)
+    assert e_got <= 1.05 * e_sep + 1e-7
+    assert worst <= 8 * 2.0 ** -11
+    none = ops.block_head(x, None, None, 1e-5, w, None)
+    plain = ops.linear(ops.layer_norm(x, None, None, 1e-5, out_dtype=torch.float16), w, None,
+                       out_dtype=torch.float16)
+    assert float((none.double() - plain.double()).abs().max()) <= 8 * 2.0 ** -11 * float(
+        plain.double().abs().max())

@@ -91,6 +91,10 @@ _SIGNATURES = {
         [C.c_int, C.c_int, _P, _I64, _P, _I64, _P, _P, C.c_float, _P, _I64, _I64, _I64, _I64,
          C.c_int, _P],
     ),
+    "mi355_block_head": (
+        C.c_int,
+        [C.c_int, _P, _I64, _P, _P, C.c_float, _P, _P, _P, _I64, _I64, _I64, _P],
+    ),
     "mi355_block_tail": (
         C.c_int,
         [C.c_int, _P, _I64, _P, _I64, _P, _I64, _P, _P, _P, _P, C.c_float, _P, _P, _P, _P, _I64,

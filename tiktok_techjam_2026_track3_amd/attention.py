@@ -333,7 +333,8 @@ class SelfAttention(nn.Module):
         extra "norm" stage before "qkv".
         """
         mark = marks or (lambda _stage: None)
-        ctx, x2, row_valid, w_o, b_o = self._normed_context(x, norm, valid_token_mask, causal, mark)
+        ctx, x2, row_valid, w_o, b_o = self._normed_context(x, norm, valid_token_mask, causal, mark,
+                                                            fused=marks is None)
         mark("out")
         out = ops.linear(ctx, w_o, b_o, row_valid=row_valid, out_dtype=x.dtype, residual=x2)
         mark("end")
@@ -341,9 +342,11 @@ class SelfAttention(nn.Module):
 
     def _normed_context(self, x: torch.Tensor, norm: nn.LayerNorm,
                         valid_token_mask: Optional[torch.Tensor], causal: bool,
-                        mark: Callable[[str], None]):
+                        mark: Callable[[str], None], fused: bool):
         """norm, QKV projection and attention of ``forward_residual``: ``(ctx [T, d], x [T, d],
-        row_valid, W_o, b_o)``, what the out projection and the residual need."""
+        row_valid, W_o, b_o)``, what the out projection and the residual need. ``fused``: narrow
+        fp32 models on fp16 operands run norm and projection as one launch (``ops.block_head``:
+        1 280 000 x 128 rows 590 -> 370 us), so no "norm" / "qkv" stages are marked."""
         B, S = self._check_input(x)
         d = self.d_model
         if tuple(norm.normalized_shape) != (d,):
@@ -366,11 +369,20 @@ class SelfAttention(nn.Module):
             qkv = ops.layernorm_linear(x2, wf, colsum, bf, norm.eps, out_dtype=core,
                                        key_bounds=kbt)
         else:
-            mark("norm")
-            h = ops.layer_norm(x2, w_n.detach() if w_n is not None else None,
-                               b_n.detach() if b_n is not None else None, norm.eps, out_dtype=op)
-            mark("qkv")
-            qkv = ops.linear(h, w_qkv, b_qkv, out_dtype=core, key_bounds=kbt)
+            w_n = w_n.detach() if w_n is not None else None
+            b_n = b_n.detach() if b_n is not None else None
+            if (fused and x.dtype == torch.float32 and op == core == torch.float16
+                    and d in ops.BLOCK_HEAD_SIZES and B * S >= ops.BLOCK_HEAD_MIN_ROWS
+                    and all(t is None or (t.is_contiguous() and t.data_ptr() % 16 == 0)
+                            for t in (x2, w_n, b_n))):
+                # (its projection writes no key bounds; a plan for them is never met here: they
+                # need K columns in multiples of 256)
+                qkv = ops.block_head(x2, w_n, b_n, norm.eps, w_qkv, b_qkv)
+            else:
+                mark("norm")
+                h = ops.layer_norm(x2, w_n, b_n, norm.eps, out_dtype=op)
+                mark("qkv")
+                qkv = ops.linear(h, w_qkv, b_qkv, out_dtype=core, key_bounds=kbt)
         q, k, v = self._qkv_views(qkv, B, S)
         mark("attn")
         ctx = self._attend(q, k, v, causal, key_valid, kbt)

@@ -375,6 +375,43 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: Optional[t
     return out
 
 
+# d_model that block_head takes: the packed QKV weight resident in LDS
+BLOCK_HEAD_SIZES = frozenset((32, 64, 128))
+# ... and the rows from which it pays: every CU's work-group stages the whole weight (96 KB at d
+# 128) for its rows, which on 8192 rows cost more than the launch saved (4-layer model 162 -> 178 us)
+BLOCK_HEAD_MIN_ROWS = 65536
+
+
+def block_head(x: torch.Tensor, norm_w: Optional[torch.Tensor], norm_b: Optional[torch.Tensor],
+               eps: float, w_qkv: torch.Tensor, b_qkv: Optional[torch.Tensor]) -> torch.Tensor:
+    """``linear(layer_norm(x), w_qkv, b_qkv)`` with fp16 operands of a narrow block in one launch:
+    ``x`` ([M, d], fp32 or fp16, unit column stride) gives fp16 [M, 3 d]; the normalised rows are
+    rounded to fp16 as ``layer_norm`` with an fp16 output rounds them. ``w_qkv`` is contiguous fp16
+    [3 d, d], ``b_qkv`` fp32, the norm's parameters of x's type; d must be in
+    ``BLOCK_HEAD_SIZES``."""
+    _on_gpu(x, norm_w, norm_b, w_qkv, b_qkv)
+    if x.dim() != 2 or x.stride(1) != 1:
+        raise ValueError("block_head expects a 2-D x with unit column stride")
+    M, d = x.shape
+    if x.dtype not in (torch.float32, torch.float16):
+        raise TypeError("x must be fp32 or fp16")
+    if tuple(w_qkv.shape) != (3 * d, d) or w_qkv.dtype != torch.float16 or not w_qkv.is_contiguous():
+        raise ValueError(f"w_qkv must be contiguous fp16 [{3 * d}, {d}]")
+    for t, n, dt in ((b_qkv, 3 * d, torch.float32), (norm_w, d, x.dtype), (norm_b, d, x.dtype)):
+        if t is not None and (tuple(t.shape) != (n,) or t.dtype != dt or not t.is_contiguous()):
+            raise ValueError("b_qkv must be contiguous fp32 and the norm's parameters of x's dtype")
+    y = torch.empty((M, 3 * d), device=x.device, dtype=torch.float16)
+
+    def ptr(t):
+        return t.data_ptr() if t is not None else 0
+
+    st = _lib.lib().mi355_block_head(_lib.dtype_code(x.dtype), x.data_ptr(), x.stride(0), ptr(norm_w),
+                                     ptr(norm_b), float(eps), w_qkv.data_ptr(), ptr(b_qkv),
+                                     y.data_ptr(), y.stride(0), M, d, _stream(x))
+    _lib.check("mi355_block_head", st)
+    return y
+
+
 # (d_model, ffn_dim) that block_tail takes: three fp16 weight matrices resident in LDS
 BLOCK_TAIL_SIZES = frozenset(((32, 32), (32, 64), (32, 128), (64, 64), (64, 128), (128, 64),
                               (128, 128)))

@@ -130,7 +130,7 @@ def _takes_tail(block: nn.Module, x: torch.Tensor) -> bool:
             and not attn.folds_norm(x.dtype, x.numel())
             and (attn.d_model, block.ffn_in.out_features) in ops.BLOCK_TAIL_SIZES
             and all(p is None or (p.data_ptr() % 16 == 0 and p.is_contiguous())
-                    for p in (block.norm2.weight, block.norm2.bias)))
+                    for p in (x, block.norm2.weight, block.norm2.bias)))
 
 
 def block_forward(block: nn.Module, x: torch.Tensor, valid_token_mask: Optional[torch.Tensor],
@@ -158,7 +158,8 @@ def block_forward(block: nn.Module, x: torch.Tensor, valid_token_mask: Optional[
     _, row_valid = attn._resolve_mask(valid_token_mask, B, S, x.device)
 
     if marks is None and _takes_tail(block, x):
-        ctx, x2, _, w_o, b_o = attn._normed_context(x, block.norm1, valid_token_mask, causal, mark)
+        ctx, x2, _, w_o, b_o = attn._normed_context(x, block.norm1, valid_token_mask, causal, mark,
+                                                    fused=True)
         w2, b2 = _norm_params(block.norm2, x)
         w_in, b_in, w_out, b_out = _ffn_weights(block, torch.float16, x.device)
         y = ops.block_tail(ctx, x2, w_o, b_o, w2, b2, block.norm2.eps, w_in, b_in, w_out, b_out,
@@ -169,7 +170,8 @@ def block_forward(block: nn.Module, x: torch.Tensor, valid_token_mask: Optional[
         if stage != "end":
             mark(stage)
 
-    x1 = attn.forward_residual(x, block.norm1, valid_token_mask, causal, marks=inner)
+    x1 = attn.forward_residual(x, block.norm1, valid_token_mask, causal,
+                               marks=inner if marks is not None else None)
     x1 = x1.reshape(B * S, d)
     w2, b2 = _norm_params(block.norm2, x)
     # the FFN's operand dtype: the model's, or fp16 for fp32 models with an fp16 attention core
