@@ -99,12 +99,12 @@ TRAFFIC_FILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profile
 def stage_kernels(w, stage: str, core_dtype):
     """Kernel families the stage launches on this build: the attention stage runs the matrix-core
     kernel (with its key-norm bound pass) for 16-bit cores at head dims 32 / 64 / 128, else the
-    vector-ALU kernel; the projections run the GEMM kernels."""
+    tiled, the fp32 or (small problems) the vector-ALU kernel; the projections run the GEMM kernels."""
     import torch
     if stage == "attn":
         if core_dtype in (torch.float16, torch.bfloat16) and w.head_dim in (32, 64, 128):
             return ("attn_fwd_mfma", "attn_key_bound")
-        return ("attn_fwd_valu",)
+        return ("attn_fwd_tiled", "attn_fwd_f32", "attn_fwd_valu")
     return ("gemm_kernel", "gemm_splitk", "gemm_f32_splitk", "layernorm_stats")
 
 

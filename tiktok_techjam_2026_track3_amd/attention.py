@@ -44,7 +44,8 @@ from .graph import AutoGraph, version_of
 
 _CACHE_KEYS = ("_mi355_pack", "_mi355_lnpack")
 
-# head dims of the fp16 / bf16 matrix-core attention kernel (the others run on vector ALUs)
+# head dims of the fp16 / bf16 attention kernel that fp32 models take through their fp16 core (at
+# the other head dims they keep an fp32 core)
 MFMA_HEAD_DIMS = (32, 64, 128)
 
 
@@ -63,7 +64,7 @@ class SelfAttention(nn.Module):
     # fp16 MFMA kernel -- the fp16 tiles the reference's fast route uses for fp32 models
     # (Project/submission/dispatcher_region.py:1017-1091); the out projection reads the fp16
     # context with an fp16 copy of its weight and returns fp32. torch.float32 keeps the core
-    # in fp32 (the vector-ALU kernel).
+    # in fp32 (fp32 matrix instructions or, for few query tiles, the vector-ALU kernel).
     fp32_core_dtype = torch.float16
     # forward_residual folds the LayerNorm into the QKV projection (row statistics pass + the
     # projection's epilogue) for fp32 and fp16 inputs; False runs the LayerNorm kernel and a
