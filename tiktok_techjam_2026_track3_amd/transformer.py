@@ -122,13 +122,14 @@ def _takes_tail(block: nn.Module, x: torch.Tensor) -> bool:
     weights that fit the kernel together. There the separate launches are bound by their passes
     over memory and, at small batches, by their number: 1 280 000 x 128 fp32 rows 1425 -> 430 us."""
     attn = block.attention
-    return (type(attn).forward_residual is SelfAttention.forward_residual
-            and type(attn)._normed_context is SelfAttention._normed_context
+    # first what most blocks fail: a small layer's forward is bound by its host code
+    return (not attn.folds_norm(x.dtype, x.numel())
             and x.dtype in (torch.float32, torch.float16)
+            and (attn.d_model, block.ffn_in.out_features) in ops.BLOCK_TAIL_SIZES
+            and type(attn).forward_residual is SelfAttention.forward_residual
+            and type(attn)._normed_context is SelfAttention._normed_context
             and attn.operand_dtype(x.dtype, x.numel()) == torch.float16
             and attn.core_dtype(x.dtype) == torch.float16
-            and not attn.folds_norm(x.dtype, x.numel())
-            and (attn.d_model, block.ffn_in.out_features) in ops.BLOCK_TAIL_SIZES
             and all(p is None or (p.data_ptr() % 16 == 0 and p.is_contiguous())
                     for p in (x, block.norm2.weight, block.norm2.bias)))
 
