@@ -610,6 +610,28 @@ def test_block_tail_unsupported_size_and_nulls(gpu):
     assert torch.all(out == 0)
 
 
+@pytest.mark.parametrize("which", ["attention.out_proj", "ffn_in", "ffn_out"])
+def test_narrow_block_takes_unaligned_biases(gpu, which):
+    """A bias that is a view into a flat buffer, 4 bytes past a 16-byte boundary: the separate
+    launches take it, so the block gives what they give."""
+    from tiktok_techjam_2026_track3_amd.transformer import TransformerBlock, _takes_tail, block_forward
+    torch.manual_seed(3)
+    blk = TransformerBlock(128, 4, 128).to(gpu).eval()
+    x = torch.randn(3, 37, 128, device=gpu)
+    with torch.inference_mode():
+        assert _takes_tail(blk, x)
+        want = block_forward(blk, x, None, False, marks=lambda stage: None)
+    lin = blk.get_submodule(which)
+    flat = torch.empty(132, device=gpu)
+    flat[1:129] = lin.bias.detach()
+    lin.bias = torch.nn.Parameter(flat[1:129])
+    assert lin.bias.data_ptr() % 16 == 4
+    with torch.inference_mode():
+        assert not _takes_tail(blk, x)
+        got = block_forward(blk, x, None, False)
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 @pytest.mark.parametrize("d", [32, 64, 128])
 @pytest.mark.parametrize("M", [1, 63, 65, 1000, 65536 + 131])

@@ -426,7 +426,7 @@ extern "C" int mi355_block_tail(int dtype, const void* ctx, int64_t ldc, const v
   if (dtype != MI355_F32 && dtype != MI355_F16) return MI355_E_BAD_DTYPE;
   if (M == 0) return MI355_OK;
   if (!ctx || !X || !Y || !W_o || !W_in || !W_out) return MI355_E_NULL_POINTER;
-  if (!(eps >= 0.f) || ldc < d_model || ldx < d_model || ldy < d_model) return MI355_E_BAD_SIZE;
+  if (ldc < d_model || ldx < d_model || ldy < d_model) return MI355_E_BAD_SIZE;
   // 16-byte accesses of the context, weights and biases, four elements of the rest
   const int64_t vx = dtype == MI355_F32 ? 15 : 7;
   auto off = [](const void* p, int64_t mask) { return (reinterpret_cast<uintptr_t>(p) & mask) != 0; };
@@ -449,7 +449,7 @@ extern "C" int mi355_block_head(int dtype, const void* X, int64_t ldx, const voi
   if (dtype != MI355_F32 && dtype != MI355_F16) return MI355_E_BAD_DTYPE;
   if (M == 0) return MI355_OK;
   if (!X || !W_qkv || !Y) return MI355_E_NULL_POINTER;
-  if (!(eps >= 0.f) || ldx < d_model || ldy < 3 * d_model) return MI355_E_BAD_SIZE;
+  if (ldx < d_model || ldy < 3 * d_model) return MI355_E_BAD_SIZE;
   const int64_t vx = dtype == MI355_F32 ? 15 : 7;
   auto off = [](const void* p, int64_t mask) { return (reinterpret_cast<uintptr_t>(p) & mask) != 0; };
   if (ldx % 4 || ldy % 8 || off(X, vx) || off(gamma, vx) || off(beta, vx) || off(W_qkv, 15) ||

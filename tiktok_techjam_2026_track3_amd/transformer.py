@@ -131,7 +131,12 @@ def _takes_tail(block: nn.Module, x: torch.Tensor) -> bool:
             and attn.operand_dtype(x.dtype, x.numel()) == torch.float16
             and attn.core_dtype(x.dtype) == torch.float16
             and all(p is None or (p.data_ptr() % 16 == 0 and p.is_contiguous())
-                    for p in (x, block.norm2.weight, block.norm2.bias)))
+                    for p in (x, block.norm2.weight, block.norm2.bias))
+            # read where they are if they have the kernel's type already (fp32 biases): parameters
+            # that are views into one flat buffer may stand at any 4 bytes, and ops.linear takes those
+            and all(p is None or p.data_ptr() % 16 == 0
+                    for lin in (attn.out_proj, block.ffn_in, block.ffn_out)
+                    for p in (lin.bias, lin.weight if x.dtype == torch.float16 else None)))
 
 
 def block_forward(block: nn.Module, x: torch.Tensor, valid_token_mask: Optional[torch.Tensor],
