@@ -665,3 +665,44 @@ def test_block_head(gpu, dtype, d, M):
                        out_dtype=torch.float16)
     assert float((none.double() - plain.double()).abs().max()) <= 8 * 2.0 ** -11 * float(
         plain.double().abs().max())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("d,ffn", [(32, 32), (32, 64), (32, 128), (64, 64), (64, 128), (128, 64),
+                                   (128, 128)])
+def test_narrow_kernels_give_the_separate_launches_bits(gpu, dtype, d, ffn):
+    """block_head and block_tail sum the norms and form the products in the order of the launches
+    they stand for (tiled GEMMs at this many rows): the same bits, but where a GELU output is
+    rounded to fp16 through fp32 instead of at once. That takes an fp32 product on a tie of fp16
+    (one in 2^13) and moves that output by a step, so at most ffn 2^-13 of the rows by a step of
+    max |g| times |w_out|."""
+    from tiktok_techjam_2026_track3_amd import ops
+    g = torch.Generator(device=gpu).manual_seed(d + ffn)
+
+    def r(*s, scale=1.0):
+        return torch.randn(*s, generator=g, device=gpu) * scale
+
+    M, half = 65536 + 131, torch.float16
+    x, gm, bt = (r(M, d) * 3 + 1.5).to(dtype), (r(d) * 0.3 + 1).to(dtype), (r(d) * 0.2).to(dtype)
+    x[:1000] *= 100
+    print(f"narrow bits {dtype} d={d} ffn={ffn}", flush=True)
+    w, b = r(3 * d, d, scale=d ** -0.5).half(), r(3 * d)
+    h = ops.layer_norm(x, gm, bt, 1e-5, out_dtype=half)
+    assert torch.equal(ops.block_head(x, gm, bt, 1e-5, w, b), ops.linear(h, w, b, out_dtype=half))
+    ctx, mask = r(M, d).half(), r(M) > -0.5
+    w_o, w_in, w_out = (r(n, k, scale=k ** -0.5).half() for n, k in ((d, d), (ffn, d), (d, ffn)))
+    b_o, b_in, b_out = r(d), r(ffn), r(d)
+    for m in (None, mask):
+        x1 = ops.linear(ctx, w_o, b_o, row_valid=m, residual=x, out_dtype=dtype)
+        h = ops.layer_norm(x1, gm, bt, 1e-5, out_dtype=half)
+        f = ops.linear(h, w_in, b_in, gelu=True, out_dtype=half)
+        want = ops.linear(f, w_out, b_out, residual=x1, row_valid=m, zero_masked_rows=True,
+                          out_dtype=dtype)
+        got = ops.block_tail(ctx, x, w_o, b_o, gm, bt, 1e-5, w_in, b_in, w_out, b_out, row_valid=m)
+        rows = float((got != want).any(1).double().mean())
+        step = 2.0 ** -10 * float(f.abs().max()) * float(w_out.abs().max())
+        print(f"  rows that differ {rows:.3g}", flush=True)
+        assert rows <= ffn * 2.0 ** -13
+        # (and the rounding of y itself)
+        ulp = 2.0 ** -10 if dtype == half else 2.0 ** -23
+        assert torch.all((got.double() - want.double()).abs() <= step + ulp * want.double().abs())

@@ -8,11 +8,14 @@
 //
 // A wave owns RT blocks of 16 rows from the context to the output and nothing crosses waves. Each
 // product is formed transposed on 16x16x32 MFMAs (A = 16 weight rows from LDS, B = 16 rows of the
-// activations), which leaves lane l four consecutive features 4 (l / 16) .. of row l % 16 per
-// block. That is the residual's and the output's layout (16-byte accesses), a row's sums are one
-// exchange over four lanes, and two blocks of it are the next product's B operand once that weight
-// is stored with its k order permuted to match (stage_weight): x1, the normalised row and the GELU
-// output stay in registers. The rounding points are those of the separate launches. [1280000, 128]
+// activations), which leaves lane l four rows 4 (l / 16) .. of the block for activation row l % 16.
+// A block's weight rows are free to choose: with those of stage_weight two blocks leave a lane 8
+// consecutive features, 8 (l / 16) .. of 32, which is the next product's B operand as it stands.
+// x1, the normalised row and the GELU output stay in registers, and a row's sums are one exchange
+// over four lanes. Rounding points, the products' order and the norm's sums are those of the
+// separate launches (where the out projection is not the split-K kernel's); one GELU output in
+// millions differs by an fp16 step: there the compiler rounds x Phi(x) to fp16 at once
+// (v_fma_mixlo_f16), here in pairs after fp32, and forcing the former cost 3%. [1280000, 128]
 // fp32: the four launches 1425 us, this one 430; the official 4-layer model over 10 000 sequences
 // 10.42 -> 5.49 ms, over 64 0.210 -> 0.162.
 #include <type_traits>
@@ -45,22 +48,21 @@ MI355_DEVINL int swz_w(int r) {
     return (4 - (r >> 2)) & 3;
 }
 
-// W [N, K] into LDS, rows of K / 8 swizzled chunks. PERM: chunk q of a 32-wide k-step holds k
-// 4 q .. + 3 and 16 + 4 q .. + 3 of it instead of 8 q .. + 7 (see the head of the file).
+// Feature of row r (4 q + i of block r / 16) of the products' N dimension with PERM: 8 q + 4 b + i of
+// the 32 that blocks 2 s + b share.
+MI355_DEVINL int feature_of(int r) { return r / 32 * 32 + r % 16 / 4 * 8 + r % 32 / 16 * 4 + r % 4; }
+
+// W [N, K] into LDS, rows of K / 8 swizzled chunks; LDS row r is W's row r, or (PERM) feature_of(r)
 template <int N, int K, int NT, bool PERM>
 MI355_DEVINL void stage_weight(u32x4* lds, const _Float16* __restrict__ w) {
-  constexpr int NCH = K / 8;
-  for (int i = threadIdx.x; i < N * NCH; i += NT) {
+  constexpr int NCH = K / 8, STEPS = (N * NCH + NT - 1) / NT;
+#pragma unroll 8
+  for (int it = 0; it < STEPS; ++it) {  // unrolled: loads in flight together
+    const int i = it * NT + static_cast<int>(threadIdx.x);
+    if (N * NCH % NT != 0 && i >= N * NCH) break;
     const int r = i / NCH, c = i % NCH;
-    u32x4 v;
-    if constexpr (PERM) {
-      const _Float16* src = w + r * K + c / 4 * 32 + c % 4 * 4;
-      const u32x2 lo = *reinterpret_cast<const u32x2*>(src), hi = *reinterpret_cast<const u32x2*>(src + 16);
-      v = u32x4{lo[0], lo[1], hi[0], hi[1]};
-    } else {
-      v = *reinterpret_cast<const u32x4*>(w + r * K + c * 8);
-    }
-    lds[r * NCH + (c ^ swz_w<NCH>(r))] = v;
+    lds[r * NCH + (c ^ swz_w<NCH>(r))] =
+        *reinterpret_cast<const u32x4*>(w + (PERM ? feature_of(r) : r) * K + c * 8);
   }
 }
 
@@ -68,6 +70,43 @@ MI355_DEVINL float quad_add(float v) {  // over lanes l, l ^ 16, l ^ 32, l ^ 48
   v = pair_sum(v);
   const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// v[0 .. N) summed as a butterfly over N lanes would: halves onto each other, N a power of two
+template <int N>
+MI355_DEVINL float halves_sum(const float (&v)[N]) {
+  float t[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) t[i] = v[i];
+#pragma unroll
+  for (int h = N / 2; h >= 1; h /= 2)
+#pragma unroll
+    for (int i = 0; i < h; ++i) t[i] += t[i + h];
+  return t[0];
+}
+
+// Sum of term(x) over a row whose lanes (q = l / 16) hold elements 32 s + 8 q + 4 j + e in x[s][j][e],
+// in the LayerNorm kernel's order: the elements of a 16-byte vector in turn (fp32: j's four, fp16:
+// all eight), then the vectors' tree -- offsets 16 .. 1 over vectors 8 s + 2 q + j or 4 s + q.
+template <typename T, int S, typename X, typename F>
+MI355_DEVINL float row_sum(const X& x, F&& term) {
+  constexpr int NV = sizeof(T) == 4 ? 2 : 1;
+  float total = 0.f;
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    float part[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      part[s] = 0.f;
+#pragma unroll
+      for (int j = v; j < (NV == 2 ? v + 1 : 2); ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) part[s] += term(x[2 * s + j][e]);
+    }
+    const float t = quad_add(halves_sum(part));
+    total = v == 0 ? t : total + t;
+  }
+  return total;
 }
 
 template <typename T>
@@ -85,7 +124,7 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void block_tail(TailArgs p) {
   static_assert(D % 32 == 0 && F % 32 == 0, "whole MFMA steps");
   constexpr int DB = D / 16, FB = F / 16, NT = NW * 64, ROWS = 16 * RT * NW;
   __shared__ u32x4 lds_o[D * D / 8], lds_1[F * D / 8], lds_2[D * F / 8];
-  stage_weight<D, D, NT, false>(lds_o, p.wo);
+  stage_weight<D, D, NT, true>(lds_o, p.wo);
   stage_weight<F, D, NT, true>(lds_1, p.w1);
   stage_weight<D, F, NT, true>(lds_2, p.w2);
   __syncthreads();
@@ -119,9 +158,10 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void block_tail(TailArgs p) {
     }
     fence();
   };
-  // features 16 fb + 4 q .. + 3 of a bias
+  // the lane's four features of block fb
+  auto feat = [&](int fb) MI355_LAMBDA_INLINE { return fb / 2 * 32 + 8 * q + fb % 2 * 4; };
   auto bias4 = [&](const float* b, int fb) MI355_LAMBDA_INLINE {
-    return b != nullptr ? *reinterpret_cast<const f32x4*>(b + 16 * fb + 4 * q) : f32x4{0.f, 0.f, 0.f, 0.f};
+    return b != nullptr ? *reinterpret_cast<const f32x4*>(b + feat(fb)) : f32x4{0.f, 0.f, 0.f, 0.f};
   };
   using cD = std::integral_constant<int, D>;
   using cF = std::integral_constant<int, F>;
@@ -149,7 +189,7 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void block_tail(TailArgs p) {
     for (int r = 0; r < RT; ++r)
 #pragma unroll
       for (int fb = 0; fb < DB; ++fb)
-        x1[r][fb] = load4f(static_cast<const T*>(p.x) + row[r] * p.ldx + 16 * fb + 4 * q);
+        x1[r][fb] = load4f(static_cast<const T*>(p.x) + row[r] * p.ldx + feat(fb));
 
     // x1 = x + out_proj(ctx): the projection rounded to x's type, masked rows 0, then the sum
     f32x4 acc[RT][DB];
@@ -167,31 +207,23 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void block_tail(TailArgs p) {
         }
     }
     fence();
-    // norm2, as the LayerNorm kernel: mean and biased variance by two passes over the registers
+    // norm2, as the LayerNorm kernel: mean and biased variance by two passes over the registers, in its
+    // order of sums
     f16x8 h[RT][D / 32];
     float mean[RT], rstd[RT];
 #pragma unroll
     for (int r = 0; r < RT; ++r) {
-      float sum = 0.f;
-#pragma unroll
-      for (int fb = 0; fb < DB; ++fb) sum += (x1[r][fb][0] + x1[r][fb][1]) + (x1[r][fb][2] + x1[r][fb][3]);
-      mean[r] = quad_add(sum) / static_cast<float>(D);
-      float sq = 0.f;
-#pragma unroll
-      for (int fb = 0; fb < DB; ++fb)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float d = x1[r][fb][e] - mean[r];
-          sq += d * d;
-        }
-      rstd[r] = 1.0f / sqrtf(quad_add(sq) / static_cast<float>(D) + p.eps);
+      const float mu = row_sum<T, D / 32>(x1[r], [](float v) { return v; }) / static_cast<float>(D);
+      const float sq = row_sum<T, D / 32>(x1[r], [mu](float v) { return (v - mu) * (v - mu); });
+      mean[r] = mu;
+      rstd[r] = 1.0f / sqrtf(sq / static_cast<float>(D) + p.eps);
     }
 #pragma unroll
     for (int fb = 0; fb < DB; ++fb) {
       fence();
       f32x4 gm = {1.f, 1.f, 1.f, 1.f}, bt = {0.f, 0.f, 0.f, 0.f};
-      if (p.gamma) gm = load4f(static_cast<const T*>(p.gamma) + 16 * fb + 4 * q);
-      if (p.beta) bt = load4f(static_cast<const T*>(p.beta) + 16 * fb + 4 * q);
+      if (p.gamma) gm = load4f(static_cast<const T*>(p.gamma) + feat(fb));
+      if (p.beta) bt = load4f(static_cast<const T*>(p.beta) + feat(fb));
 #pragma unroll
       for (int r = 0; r < RT; ++r)
 #pragma unroll
@@ -230,7 +262,7 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void block_tail(TailArgs p) {
           const float v = to_f32(from_f32<T>(acc[r][fb][e] + b[e])) + x1[r][fb][e];
           w[e] = from_f32<T>(valid[r] ? v : 0.f);
         }
-        if (in[r]) *reinterpret_cast<t4*>(static_cast<T*>(p.y) + row[r] * p.ldy + 16 * fb + 4 * q) = w;
+        if (in[r]) *reinterpret_cast<t4*>(static_cast<T*>(p.y) + row[r] * p.ldy + feat(fb)) = w;
       }
     }
   }
@@ -273,34 +305,21 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void block_head(HeadArgs p) {
       in[r] = row[r] < p.M;
       if (!in[r]) row[r] = p.M - 1;  // a real row, computed again and not stored
     }
-    f32x4 xv[RT][D / 32][2];
+    f32x4 xv[RT][D / 16];
 #pragma unroll
     for (int r = 0; r < RT; ++r)
 #pragma unroll
       for (int s = 0; s < D / 32; ++s)
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-          xv[r][s][j] = load4f(static_cast<const T*>(p.x) + row[r] * p.ldx + 32 * s + 8 * q + 4 * j);
+          xv[r][2 * s + j] = load4f(static_cast<const T*>(p.x) + row[r] * p.ldx + 32 * s + 8 * q + 4 * j);
     float mean[RT], rstd[RT];
 #pragma unroll
     for (int r = 0; r < RT; ++r) {
-      float sum = 0.f;
-#pragma unroll
-      for (int s = 0; s < D / 32; ++s)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) sum += (xv[r][s][j][0] + xv[r][s][j][1]) + (xv[r][s][j][2] + xv[r][s][j][3]);
-      mean[r] = quad_add(sum) / static_cast<float>(D);
-      float sq = 0.f;
-#pragma unroll
-      for (int s = 0; s < D / 32; ++s)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float d = xv[r][s][j][e] - mean[r];
-            sq += d * d;
-          }
-      rstd[r] = 1.0f / sqrtf(quad_add(sq) / static_cast<float>(D) + p.eps);
+      const float mu = row_sum<T, D / 32>(xv[r], [](float v) { return v; }) / static_cast<float>(D);
+      const float sq = row_sum<T, D / 32>(xv[r], [mu](float v) { return (v - mu) * (v - mu); });
+      mean[r] = mu;
+      rstd[r] = 1.0f / sqrtf(sq / static_cast<float>(D) + p.eps);
     }
 #pragma unroll
     for (int s = 0; s < D / 32; ++s)
@@ -314,7 +333,7 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void block_head(HeadArgs p) {
         for (int r = 0; r < RT; ++r)
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            h[r][s][4 * j + e] = from_f32<_Float16>((xv[r][s][j][e] - mean[r]) * rstd[r] * gm[e] + bt[e]);
+            h[r][s][4 * j + e] = from_f32<_Float16>((xv[r][2 * s + j][e] - mean[r]) * rstd[r] * gm[e] + bt[e]);
       }
     // q, k and v in turn: D features each
 #pragma unroll 1
