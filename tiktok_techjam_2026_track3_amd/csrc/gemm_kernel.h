@@ -316,7 +316,7 @@ __global__ __launch_bounds__(WM* WN * 64, (WM * WN <= 4 && BM < 256) ? MI355_GEM
       if (rd) {
         if constexpr (DB) {
           // W and A fragments in the order the next slice uses them: W 0, every A, W 1 ..
-          constexpr int EVERY = NPOS / (TM + TN) > 1 ? NPOS / (TM + TN) : 1;
+          constexpr int EVERY = EPM > 1 ? 2 : NPOS / (TM + TN) > 1 ? NPOS / (TM + TN) : 1;
           constexpr int PER = (TM + TN + NPOS - 1) / NPOS;
           if (i % EVERY == 0) {
 #pragma unroll
@@ -495,12 +495,14 @@ __global__ __launch_bounds__(WM* WN * 64, (WM * WN <= 4 && BM < 256) ? MI355_GEM
       if (!(v < nk || (nxt && has_next))) r.a[2] = r.w[2] = 0u;
       return r;
     };
-    // load l of a step after the MFMA at position l * NPOS / NLD of the slice that frees its slot
-    static_assert(NLD <= NPOS, "a step's loads between the MFMAs of one slice");
+    // load l of a step after the MFMA at position l * SPAN / NLD of the slice that frees its slot
+    // (fp32, whose slice is four times as long: of its first half)
+    constexpr int SPAN = EPM > 1 ? NPOS / 2 : NPOS;
+    static_assert(NLD <= SPAN, "a step's loads between the MFMAs of one slice");
     auto load_at = [&](const StepSrc& src, const int slot, auto ic) MI355_LAMBDA_INLINE {
       constexpr int i = decltype(ic)::value;
-      constexpr int l = (i * NLD + NPOS - 1) / NPOS;  // first load at position i or after it
-      if constexpr (l < NLD && l * NPOS / NLD == i) {
+      constexpr int l = (i * NLD + SPAN - 1) / SPAN;  // first load at position i or after it
+      if constexpr (l < NLD && l * SPAN / NLD == i) {
         load_one(slot, src, std::integral_constant<int, l>{});
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -510,13 +512,27 @@ __global__ __launch_bounds__(WM* WN * 64, (WM * WN <= 4 && BM < 256) ? MI355_GEM
     auto k_loop = [&]() MI355_LAMBDA_INLINE {
 #pragma unroll
       for (int f = 0; f < TM + TN; ++f) read_frag(0, 0, 0, f);
-#pragma unroll 1
-      for (int kt = 0; kt < nk; ++kt) {
-        const int slot = kt & 1;
+      auto step = [&](const int kt, const int slot) MI355_LAMBDA_INLINE {
         const StepSrc src = src_of(kt + 2);
         slice(0, slot, 1, true, [](auto) {});
         ring_barrier();
         slice(1, slot ^ 1, 0, true, [&](auto i) MI355_LAMBDA_INLINE { load_at(src, slot, i); });
+      };
+      int kt = 0;
+      if constexpr (EPM > 1) {
+        // fp32: both slots unrolled. With kt & 1 every read's LDS address and every load's source
+        // was formed anew per step, about 30 vector operations beside 128 MFMAs: 8192 x 4096 x 4096
+        // 1969 -> 1899 us (1884 with the reads after every second MFMA and the loads in the slice's
+        // first half), 2048^3 140 -> 130; the former kernel on 32x32 blocks 1880 and 131
+#pragma unroll 1
+        for (; kt + 2 <= nk; kt += 2) {
+          step(kt, 0);
+          step(kt + 1, 1);
+        }
+        if (kt < nk) step(kt, 0);
+      } else {
+#pragma unroll 1
+        for (; kt < nk; ++kt) step(kt, kt & 1);
       }
     };
     {
