@@ -888,6 +888,28 @@ def test_attention_f32_mfma_edges(gpu, hd, B, Sq, Sk):
                         packed=True)
 
 
+@pytest.mark.parametrize("hd,n,Sq,Sk,causal", [
+    (8, 382, 64, 70, False), (8, 384, 64, 70, False),       # work-groups of two waves
+    (8, 638, 65, 65, True), (8, 640, 65, 65, True),
+    (16, 260, 230, 63, False), (16, 260, 231, 63, False),   # nine tenths of a 256-query tile
+    (16, 260, 217, 217, True), (16, 260, 218, 218, True),   # causal: 85 % of it
+    (48, 260, 116, 31, False), (48, 260, 116, 32, False), (64, 260, 65, 63, False), (64, 260, 65, 64, False),
+    (32, 130, 191, 191, True), (32, 130, 192, 192, True),   # causal: three quarters of two tiles
+    (96, 260, 84, 64, False), (96, 260, 85, 64, False),     # two thirds of a tile
+    (128, 260, 128, 128, True), (80, 130, 231, 231, True),
+    (256, 260, 89, 64, False), (256, 260, 90, 64, False),   # 0.7 of one
+    (192, 130, 127, 127, True), (192, 130, 128, 128, True),
+    (256, 260, 65, 256, False), (256, 260, 65, 257, False), (64, 260, 300, 200, True),
+])
+def test_attention_f32_both_sides_of_the_rule(gpu, hd, n, Sq, Sk, causal):
+    """Shapes next to each line of mi355_internal_attn_f32_wins: the vector-ALU kernel on one side,
+    attn_fwd_f32 on the other, both against fp64, with and without a key mask."""
+    kv = torch.rand(n // 2, Sk, generator=torch.Generator().manual_seed(Sk)) > 0.3
+    kv[:, 0] = True
+    for mask in (None, kv):
+        _attn_check(gpu, torch.float32, n // 2, 2, Sq, Sk, hd, causal, seed=hd + Sq, key_valid=mask)
+
+
 # --------------------------------------------------------------- K that fills no whole step
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M,N", [(4100, 4360), (1100, 3000), (600, 1100)])

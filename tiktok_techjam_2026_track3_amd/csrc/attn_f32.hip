@@ -346,14 +346,53 @@ int launch_hd(const AttnArgs& a, bool causal, hipStream_t s) {
 
 }  // namespace
 
-// Enough work-groups for every CU, of at least a 64-query tile: with fewer the vector-ALU kernel,
-// which splits a query tile's keys over eight waves, is faster (8 heads of 512 at hd 64 139 against
-// 277 us; 512 heads of 16 queries and 2048 keys at hd 256 636 against 649; 512 heads of 64 at hd
-// 256 68 against 46).
+// Against the vector-ALU kernel, which splits a 16- or 32-query tile's keys over two or eight waves
+// and computes little more than the real rows, this one loses where few work-groups are left and
+// where its tiles (bm queries by 64 or 32 keys) are mostly padding; both were timed over 64-1000
+// queries, 1-4000 keys and 256-5000 work-groups per head dim (vector-ALU -> this kernel, us). The
+// lines lie where nothing that is taken was more than 3% slower:
+//   * below 64 queries or a work-group per CU (8 heads of 512 queries at hd 64: 139 -> 277);
+//   * hd 8, 16: work-groups of two waves are too few at one per CU (256 heads of 64 queries and 4000
+//     keys at hd 8 82 -> 149; 512 heads of 65 queries 241 -> 270, 800 of them 0.72 of the time);
+//   * up to hd 64: fewer than 64 keys, or 32 in full tiles of four waves (hd 32, 2048 heads of 64
+//     queries and 16 keys 0.69 of its speed; 129 queries and 32 keys 0.84, 64 keys 1.4);
+//   * above: up to 256 keys (where the other kernel's key split is the cheaper one of two waves) it
+//     has to fill two thirds of its tiles: 512 heads of 128 queries and 64 keys at hd 80 0.70 of the
+//     time, of 129 queries 0.90, of 64 queries 0.87, at 800 heads 0.86, 1.15 and 1.24; one key 2-4;
+//   * causal, up to 256 keys: half of those are skipped by 16-query steps there, by tiles here, so
+//     more of the tiles has to be real (640 causal heads of 80 at hd 64 25 -> 37, of 112 at hd 80 43
+//     -> 61, of 256 at hd 80 0.76 of the time; hd 8, 8192 heads of 128 as in the narrow-head layer
+//     0.60).
 bool mi355_internal_attn_f32_wins(const AttnTiledCall& call) {
   const AttnArgs& a = *static_cast<const AttnArgs*>(call.args);
-  const int64_t bm = 16 * groups_of(call.head_dim) * (a.Sq <= 32 * groups_of(call.head_dim) ? 2 : 4);
-  return a.Sq >= 64 && (a.Sq + bm - 1) / bm * a.H * a.B >= 256;
+  const int64_t hd = call.head_dim, bw = 16 * groups_of(hd);
+  const bool two_waves = a.Sq <= 2 * bw;
+  const int64_t bm = bw * (two_waves ? 2 : 4), tiles = (a.Sq + bm - 1) / bm, groups = tiles * a.H * a.B;
+  if (a.Sq < 64 || groups < 256) return false;
+  auto filled = [&](int64_t percent) { return 100 * a.Sq >= percent * tiles * bm; };  // query tiles
+  const int64_t keys = call.causal && a.Sq < a.Sk ? a.Sq : a.Sk;
+  if (call.causal && keys <= 256) {
+    if (hd == 8) {
+      if (!two_waves && !filled(75) && groups < 1024) return false;
+    } else if (hd == 16) {
+      if (!filled(85) || (two_waves && groups < 640)) return false;
+    } else if (hd <= 64) {
+      if (two_waves || !filled(tiles == 1 ? 90 : 75)) return false;
+    } else if (hd <= 128) {
+      if (tiles == 1 || !filled(90)) return false;
+    } else if (a.Sq < 128 || !filled(75)) {
+      return false;
+    }
+  }
+  if (hd <= 16) {
+    if (two_waves && groups < (a.Sq <= bw ? 384 : 8 * a.Sq < 7 * bm ? 640 : 0)) return false;
+    return hd == 8 || keys >= 64 || filled(90);
+  }
+  if (hd <= 64) return keys >= 64 || (keys >= 32 && filled(90) && !two_waves);
+  if (keys > 256) return true;
+  if (keys < 64 || (hd <= 128 && two_waves)) return false;
+  const int64_t bn = hd > 128 ? 32 : 64, padded = (keys + bn - 1) / bn * bn;
+  return 100 * a.Sq * keys >= (hd > 128 ? 70 : 66) * tiles * bm * padded;
 }
 
 int mi355_internal_attn_f32(const AttnTiledCall& call, hipStream_t s) {
