@@ -80,7 +80,7 @@ int mi355_gemm_bias(int in_dtype, int out_dtype, const void* A, int64_t lda, con
  * all -inf row does in the reference.
  * Supported: dtype F32, F16, BF16 with head_dim 8, 16, 32, 48, 64, 80, 96, 128, 192 or 256
  * (the benchmark's official shapes use 8, 32, 64, 128 and 256: Project/shapes.json). F16/BF16
- * run on the matrix cores (head_dim 192 and 256 with at most 8 queries and 8 keys excepted); F32
+ * run on the matrix cores (head_dim 192 and 256 with few queries or few keys excepted); F32
  * problems of at least 64 queries, enough query tiles for every CU and enough keys to fill them run
  * on the fp32 matrix instructions. The rest runs on a vector-ALU kernel with fp32 arithmetic (16-bit probabilities
  * are rounded the same way).

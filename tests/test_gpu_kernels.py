@@ -851,6 +851,21 @@ def test_attention_tiled_edges(gpu, dtype, hd, B, Sq, Sk, H):
                         packed=True)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("hd", [192, 256])
+@pytest.mark.parametrize("Sq,Sk", [(1, 9), (8, 32), (1, 33), (8, 112), (8, 113), (8, 160), (8, 161),
+                                   (9, 33), (16, 48), (16, 49), (17, 33), (33, 10), (48, 11), (64, 8),
+                                   (64, 9), (65, 4), (80, 4), (81, 4), (65, 5)])
+def test_attention_wide_heads_both_sides_of_the_rule(gpu, dtype, hd, Sq, Sk):
+    """Shapes next to each line of valu_wins_wide, with few and with many (batch, head) pairs (the
+    vector-ALU kernel's 8- and 2-wave key split), with and without a key mask."""
+    for B in (2, 300):
+        kv = torch.rand(B, Sk, generator=torch.Generator().manual_seed(Sk)) > 0.3
+        kv[:, 0] = True
+        for mask in (None, kv):
+            _attn_check(gpu, dtype, B, 4, Sq, Sk, hd, False, seed=hd + Sk, key_valid=mask)
+
+
 @pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
 @pytest.mark.parametrize("hd", [8, 48, 256])
 def test_attention_tiled_nonfinite_rows_stay_in_their_queries(gpu, hd, bad):

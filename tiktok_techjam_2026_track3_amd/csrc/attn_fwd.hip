@@ -1566,8 +1566,8 @@ int launch_valu(const AttnArgs& a, bool causal, bool kmask, hipStream_t s) {
   return launch_valu_nwk<T, HD, 8>(a, causal, kmask, s);
 }
 
-// head dims of the VALU kernel: fp32 all of them, 16-bit the two that prefer it for a handful of
-// keys (see attn_fwd_impl)
+// head dims of the VALU kernel: fp32 all of them, 16-bit the two that prefer it for few queries or
+// keys (valu_wins_wide)
 template <typename T>
 int dispatch_valu(const AttnArgs& a, int64_t hd, bool causal, bool kmask, hipStream_t s) {
   if (hd == 192) return launch_valu<T, 192>(a, causal, kmask, s);
@@ -1622,6 +1622,21 @@ int64_t redo_offset(int64_t B, int64_t H, int64_t S_k) {
 int64_t redo_flag_bytes(int64_t B, int64_t H, int64_t S_q, int64_t head_dim) {
   const int64_t bm = mfma_block_queries(head_dim);
   return B * H * ((S_q + bm - 1) / bm) * static_cast<int64_t>(sizeof(int));
+}
+
+// 16-bit head dims 192 and 256: where the vector-ALU kernel, which reads the real rows only, is faster
+// than a mostly empty tile of attn_fwd_tiled (vector-ALU -> tiled, us, at 256 unless said otherwise).
+// Up to 32 queries that one has a 32-key tile on one wave (8192 heads of 4 and 4: 32 -> 43; of 16: 103
+// -> 60) or, beyond 32 keys, 64-key tiles in the whole LDS for one busy wave of four (2048 heads of 8
+// queries and 33 keys 32 -> 54; 12000 heads and 112 keys 1.2, at 192 1.1, 128 keys 0.96 there; 160 keys
+// 1.11, but 0.84 of the time for 256 heads; 16 queries and 48 keys 1.06, 64 0.74); beyond 32 queries a
+// 128-query work-group (2048 heads of 33 queries and 8 keys 46 -> 58, 12000 of 12 keys 0.97; 64 and 8
+// keys 70 -> 75, 12 keys 0.74; 80 and 4 keys at 192 1.12, 96 0.85).
+bool valu_wins_wide(int64_t hd, int64_t pairs, int64_t S_q, int64_t S_k) {
+  if (S_q <= 8) return S_k <= 8 || (S_k > 32 && S_k <= (hd == 256 && pairs >= 1024 ? 160 : 112));
+  if (S_q <= 16) return S_k > 32 && S_k <= 48;
+  if (S_q <= 32) return false;
+  return S_k <= (S_q <= 48 ? 10 : S_q <= 64 ? 8 : S_q <= 80 ? 4 : 0);
 }
 
 int attn_fwd_impl(int dtype, const void* Q, const void* K, const void* V, void* O, int64_t B,
@@ -1686,10 +1701,7 @@ int attn_fwd_impl(int dtype, const void* Q, const void* K, const void* V, void* 
     return dispatch_valu<float>(a, head_dim, cz, kmask, s);
   }
   if (!on_mfma_kernel(dtype, head_dim)) {
-    // head dims 192 and 256 over at most 8 queries and keys: a 32-key tile is mostly padding there,
-    // and the vector-ALU kernel, which reads the real rows only, is faster (8192 heads of 4: 32
-    // against 43 us at 256; of 16: 103 against 60)
-    if (head_dim >= 192 && S_q <= 8 && S_k <= 8)
+    if (head_dim >= 192 && valu_wins_wide(head_dim, B * H, S_q, S_k))
       return dtype == MI355_F16 ? dispatch_valu<_Float16>(a, head_dim, cz, kmask, s)
                                 : dispatch_valu<__bf16>(a, head_dim, cz, kmask, s);
     return mi355_internal_attn_tiled({&a, head_dim, dtype == MI355_BF16, cz}, s);
