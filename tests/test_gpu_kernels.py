@@ -925,6 +925,41 @@ def test_attention_f32_both_sides_of_the_rule(gpu, hd, n, Sq, Sk, causal):
         _attn_check(gpu, torch.float32, n // 2, 2, Sq, Sk, hd, causal, seed=hd + Sq, key_valid=mask)
 
 
+@pytest.mark.parametrize("dtype,hd", [(torch.bfloat16, 16), (torch.float16, 48), (torch.float16, 80),
+                                      (torch.bfloat16, 96), (torch.float16, 192), (torch.float16, 256),
+                                      (torch.float32, 16), (torch.float32, 64), (torch.float32, 256)])
+@pytest.mark.parametrize("Sk", [20, 64, 100, 330])
+def test_attention_overlapping_key_rows(gpu, dtype, hd, Sk):
+    """K and V as windows over one buffer, each row a few elements after the one before it: the last
+    rows are read whole, and what follows them (here infinities, and those of the last row itself)
+    reaches no output element of another dim."""
+    ops = _ops()
+    B, Sq, H, step = 260, 70, 2, 8  # (strides are whole 16-byte groups)
+    n = (Sk - 1) * step + hd
+    pad = (n + 63) // 64 * 64 + 64
+    buf = [torch.full((B * H, pad), float("inf"), dtype=dtype) for _ in range(2)]
+    for i, t in enumerate(buf):
+        t[:, :n] = _rand((B * H, n), dtype, 5 + i)
+    buf[1][:, n - 1] = float("inf")  # the last key's last dim
+    q = _rand((B, Sq, H, hd), dtype, 9)
+
+    def windows(t):
+        return t.as_strided((B, Sk, H, hd), (H * pad, step, pad, 1))
+
+    print(f"overlapping rows {dtype} hd={hd} Sk={Sk} step={step}", flush=True)
+    out = ops.attention(q.to(gpu), windows(buf[0].to(gpu)), windows(buf[1].to(gpu))).cpu().double()
+    k, v = (windows(t).double() for t in buf)
+    v[..., -1] = 0
+    ref = OA.attention_core(q.double().transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2), hd ** -0.5,
+                            False, None).transpose(1, 2)
+    d = slice(0, hd - 1)
+    # (inf, or NaN from the vector-ALU kernel, which multiplies the last row by 0 past the end)
+    assert not torch.isfinite(out[..., -1]).any()
+    assert torch.isfinite(out[..., d]).all()
+    tol = 2e-6 if dtype == torch.float32 else 8 * UNIT[dtype]
+    assert float((out - ref)[..., d].norm()) <= tol * float(ref[..., d].norm())
+
+
 # --------------------------------------------------------------- K that fills no whole step
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M,N", [(4100, 4360), (1100, 3000), (600, 1100)])

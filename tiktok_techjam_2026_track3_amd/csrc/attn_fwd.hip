@@ -1695,13 +1695,16 @@ int attn_fwd_impl(int dtype, const void* Q, const void* K, const void* V, void* 
   const bool kmask = key_valid != nullptr;
   const bool cz = causal != 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  // K or V rows that overlap (a sequence stride below head_dim): the tiled kernels' load ranges end
+  // with whole strides; the vector-ALU kernel takes them, and an instance of attn_fwd_tiled
+  const bool overlap = a.ks1 < head_dim || a.vs1 < head_dim;
   if (dtype == MI355_F32) {
     const AttnTiledCall call = {&a, head_dim, false, cz};
-    if (mi355_internal_attn_f32_wins(call)) return mi355_internal_attn_f32(call, s);
+    if (!overlap && mi355_internal_attn_f32_wins(call)) return mi355_internal_attn_f32(call, s);
     return dispatch_valu<float>(a, head_dim, cz, kmask, s);
   }
   if (!on_mfma_kernel(dtype, head_dim)) {
-    if (head_dim >= 192 && valu_wins_wide(head_dim, B * H, S_q, S_k))
+    if (head_dim >= 192 && (overlap || valu_wins_wide(head_dim, B * H, S_q, S_k)))
       return dtype == MI355_F16 ? dispatch_valu<_Float16>(a, head_dim, cz, kmask, s)
                                 : dispatch_valu<__bf16>(a, head_dim, cz, kmask, s);
     return mi355_internal_attn_tiled({&a, head_dim, dtype == MI355_BF16, cz}, s);

@@ -54,8 +54,9 @@ MI355_DEVINL float sum8(bf16x8 f, float acc) {
   return acc;
 }
 
-// NW waves of QG groups of 32 queries of one (batch, head).
-template <typename T, int HD, int NW, int QG, int BN, int RING, bool CAUSAL>
+// NW waves of QG groups of 32 queries of one (batch, head). LAP: K or V rows that overlap (a stride
+// below the row's bytes, as windows over one buffer have).
+template <typename T, int HD, int NW, int QG, int BN, int RING, bool CAUSAL, bool LAP>
 __global__ __launch_bounds__(NW * 64, 2) void attn_fwd_tiled(AttnArgs p) {
   using MF = Mfma<T>;
   using frag = typename MF::frag;
@@ -92,7 +93,10 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_fwd_tiled(AttnArgs p) {
   // row strides in bytes; the entry point guarantees that 64 rows of them fit in 32 bits
   const uint32_t kstride = static_cast<uint32_t>(p.ks1) * sizeof(T);
   const uint32_t vstride = static_cast<uint32_t>(p.vs1) * sizeof(T);
-  const uint32_t kcap = 0xffffffffu / kstride, vcap = 0xffffffffu / vstride;
+  constexpr uint32_t CAP = 0xffffffffu - (LAP ? ROWB : 0);
+  const uint32_t kcap = CAP / kstride, vcap = CAP / vstride;
+  // the load ranges end rem strides on; LAP: with the last key's row, that many bytes further
+  const uint32_t kext = LAP ? ROWB - kstride : 0u, vext = LAP ? ROWB - vstride : 0u;
 
   if constexpr (HD == 8) {
     if (tid == 0) lds[2 * RING * TILE + PAD - 1] = u32x4{0u, 0u, 0u, 0u};
@@ -133,8 +137,8 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_fwd_tiled(AttnArgs p) {
   }
   auto issue_loads = [&](int j, int s) MI355_LAMBDA_INLINE {
     const uint32_t k0 = static_cast<uint32_t>(j) * BN, rem = static_cast<uint32_t>(Sk) - k0;
-    const u32x4 kr = buffer_rsrc(Kb + static_cast<uint64_t>(k0) * kstride, rem > kcap ? 0xffffffffu : rem * kstride);
-    const u32x4 vr = buffer_rsrc(Vb + static_cast<uint64_t>(k0) * vstride, rem > vcap ? 0xffffffffu : rem * vstride);
+    const u32x4 kr = buffer_rsrc(Kb + static_cast<uint64_t>(k0) * kstride, rem > kcap ? 0xffffffffu : rem * kstride + kext);
+    const u32x4 vr = buffer_rsrc(Vb + static_cast<uint64_t>(k0) * vstride, rem > vcap ? 0xffffffffu : rem * vstride + vext);
 #pragma unroll
     for (int i = 0; i < LPW; ++i) {
       const int blk = wave + i * NW;
@@ -143,7 +147,12 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_fwd_tiled(AttnArgs p) {
       // (K rows past the end may hold anything, V rows have to be zeros: P · V multiplies them.
       // Only where the tile is all there is: a branch around every load costs the long sweeps.)
       const bool any = RING > 1 || static_cast<uint32_t>(blk * 64 / KCH) < rem;
-      if constexpr (STEP) {
+      if constexpr (LAP) {  // rows past the last key are not past the range
+        const uint32_t row = static_cast<uint32_t>(blk * 64 + lane) / KCH;
+        const uint32_t c = ((blk * 64 + lane) % KCH) ^ swz_row<KCH>(static_cast<int>(row));
+        buffer_dma_lds16(kr, row * kstride + c * 16, 0, ka);
+        buffer_dma_lds16(vr, row < rem ? row * vstride + c * 16 : 0xffff0000u, 0, va);
+      } else if constexpr (STEP) {
         if (any) buffer_dma_lds16(kr, koff[0], i * ROWS * kstride, 0, ka);
         buffer_dma_lds16(vr, voff[0], i * ROWS * vstride, 0, va);
       } else {
@@ -357,7 +366,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_fwd_tiled(AttnArgs p) {
   }
 }
 
-template <typename T, int HD, int NW, int QG, int BN = 64, int RING = 2>
+template <typename T, int HD, int NW, int QG, int BN = 64, int RING = 2, bool LAP = false>
 int launch(const AttnArgs& a0, bool causal, hipStream_t s) {
   AttnArgs a = a0;
   constexpr int BM = NW * 32 * QG;
@@ -369,9 +378,9 @@ int launch(const AttnArgs& a0, bool causal, hipStream_t s) {
   if (causal && !flat) return MI355_E_BAD_SIZE;
   if (flat) grid = dim3(static_cast<unsigned>(n), 1, 1);
   if (causal)
-    hipLaunchKernelGGL((attn_fwd_tiled<T, HD, NW, QG, BN, RING, true>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((attn_fwd_tiled<T, HD, NW, QG, BN, RING, true, LAP>), grid, block, 0, s, a);
   else
-    hipLaunchKernelGGL((attn_fwd_tiled<T, HD, NW, QG, BN, RING, false>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((attn_fwd_tiled<T, HD, NW, QG, BN, RING, false, LAP>), grid, block, 0, s, a);
   return static_cast<int>(hipGetLastError());
 }
 
@@ -382,6 +391,11 @@ int launch(const AttnArgs& a0, bool causal, hipStream_t s) {
 template <typename T, int HD>
 int launch_hd(const AttnArgs& a, bool causal, hipStream_t s) {
   constexpr bool WIDE = HD > 96;
+  // (overlapping rows of 192 and 256 go to the vector-ALU kernel, and hd 8's cannot overlap: strides
+  // are whole 16-byte groups)
+  if constexpr (HD > 8 && !WIDE) {
+    if (a.ks1 < HD || a.vs1 < HD) return launch<T, HD, 4, 1, 64, 2, true>(a, causal, s);
+  }
   if (a.Sq <= 32) {
     if (a.Sk <= 32) return launch<T, HD, 1, 1, HD == 8 ? 64 : 32, 1>(a, causal, s);
     if constexpr (!WIDE) return launch<T, HD, 1, 1>(a, causal, s);
