@@ -2,6 +2,7 @@
 and rejects invalid arguments with its documented negative status codes before touching the
 device (every call below fails argument validation, so no kernel is launched)."""
 import ctypes as C
+import os
 import re
 from pathlib import Path
 
@@ -124,6 +125,21 @@ def test_attention_argument_validation():
     assert call(B=-1) == codes["MI355_E_BAD_SIZE"]
     assert call(strides=L.i64_array((3, 64, 64))) == codes["MI355_E_ALIGNMENT"]
     assert call(B=0) == 0
+
+
+@pytest.mark.skipif(os.path.exists("/dev/kfd"), reason="would launch on made-up pointers")
+@pytest.mark.parametrize("heads,refused", [(257, False), (511, False), (513, True)])
+def test_causal_heads_up_to_the_smaller_grid(heads, refused):
+    """Wide causal heads of few queries over 113 to 256 keys: 65535 * 257 of them are more than a 1-D
+    grid of four-wave work-groups holds and fit one of two-wave work-groups, so the call is not
+    refused (it fails in the launch: there is no device here)."""
+    L = _lib()
+    codes = _status_codes()
+    fake = 1 << 20
+    st, kst = L.i64_array((192 * heads, 192 * heads, 192)), L.i64_array((0, 192, 0))
+    rc = L.lib().mi355_attn_fwd(1, fake, fake, fake, fake, 65535, heads, 1, 200, 192, st, kst, kst, st,
+                                0.1, 1, None, 0, None)
+    assert (rc == codes["MI355_E_BAD_SIZE"]) == refused
 
 
 def test_attention_workspace_argument_validation():

@@ -1707,7 +1707,12 @@ int attn_fwd_impl(int dtype, const void* Q, const void* K, const void* V, void* 
     if (head_dim >= 192 && (overlap || valu_wins_wide(head_dim, B * H, S_q, S_k)))
       return dtype == MI355_F16 ? dispatch_valu<_Float16>(a, head_dim, cz, kmask, s)
                                 : dispatch_valu<__bf16>(a, head_dim, cz, kmask, s);
-    return mi355_internal_attn_tiled({&a, head_dim, dtype == MI355_BF16, cz}, s);
+    const int rc = mi355_internal_attn_tiled({&a, head_dim, dtype == MI355_BF16, cz}, s);
+    // a causal grid is 1-D and 32-bit in threads: a few wide queries of 2^24 heads and more take half
+    // the threads there
+    if (rc != MI355_E_BAD_SIZE || head_dim < 192) return rc;
+    return dtype == MI355_F16 ? dispatch_valu<_Float16>(a, head_dim, cz, kmask, s)
+                              : dispatch_valu<__bf16>(a, head_dim, cz, kmask, s);
   }
   float* kb = nullptr;
   int* redo = nullptr;
