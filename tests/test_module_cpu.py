@@ -216,3 +216,36 @@ def test_autograph_captures_form_no_reference_cycle():
             gc.enable()
     # a switch module that no longer exists gives a sentinel no recorded value equals
     assert G._switch_values([None]) == ((G._GONE,),)
+
+
+def test_narrow_block_takes_any_module_with_weight_and_bias():
+    """Whether a narrow block runs its fused tail is read off what the separate launches read: weight
+    and bias of the FFN's projections, and a forward_residual that is the module's own (a subclass's
+    or one set on the instance is called, so the tail must not pass it by)."""
+    import types
+
+    from tiktok_techjam_2026_track3_amd.transformer import TransformerBlock, _takes_tail
+
+    class Projection(torch.nn.Module):  # no in_features / out_features
+        def __init__(self, lin):
+            super().__init__()
+            self.weight, self.bias = lin.weight, lin.bias
+
+    def aligned(blk):  # the rule asks for 16-byte aligned parameters
+        for p in blk.parameters():
+            buf = torch.zeros(p.numel() + 4)
+            at = (-buf.data_ptr() // 4) % 4
+            p.data = buf[at:at + p.numel()].view(p.shape)
+        return blk
+
+    x = torch.zeros(1, 4, 64)
+    blk = aligned(TransformerBlock(64, 2, 128))
+    blk.ffn_in, blk.ffn_out = Projection(blk.ffn_in), Projection(blk.ffn_out)
+    assert _takes_tail(blk, x)
+    own = aligned(TransformerBlock(64, 2, 128))
+    assert _takes_tail(own, x)
+    own.attention.forward_residual = lambda *a, **k: None
+    assert not _takes_tail(own, x)
+    own = aligned(TransformerBlock(64, 2, 128))
+    own.attention.forward_residual = types.MethodType(lambda self, *a, **k: None, own.attention)
+    assert not _takes_tail(own, x)

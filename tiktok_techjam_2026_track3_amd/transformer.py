@@ -125,9 +125,10 @@ def _takes_tail(block: nn.Module, x: torch.Tensor) -> bool:
     # first what most blocks fail: a small layer's forward is bound by its host code
     return (not attn.folds_norm(x.dtype, x.numel())
             and x.dtype in (torch.float32, torch.float16)
-            and (attn.d_model, block.ffn_in.out_features) in ops.BLOCK_TAIL_SIZES
-            and type(attn).forward_residual is SelfAttention.forward_residual
-            and type(attn)._normed_context is SelfAttention._normed_context
+            and (attn.d_model, block.ffn_in.weight.shape[0]) in ops.BLOCK_TAIL_SIZES
+            # (a forward_residual of the class's or the instance's own is called, not passed by)
+            and getattr(attn.forward_residual, "__func__", None) is SelfAttention.forward_residual
+            and getattr(attn._normed_context, "__func__", None) is SelfAttention._normed_context
             and attn.operand_dtype(x.dtype, x.numel()) == torch.float16
             and attn.core_dtype(x.dtype) == torch.float16
             and all(p is None or (p.data_ptr() % 16 == 0 and p.is_contiguous())
