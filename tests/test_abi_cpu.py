@@ -240,6 +240,34 @@ def test_build_refuses_lds_dma_kernels_that_use_scratch():
     B.check_no_scratch("a.hip", {k: v for k, v in usage.items() if "valu" in k})
 
 
+def test_build_refuses_inline_mfmas_without_wait_states():
+    """build.py reads the GEMM units' device assembly: a VGPR written right before an MFMA that reads
+    it, and an MFMA's result used by another instruction before it is there, along the text and over a
+    loop's back edge."""
+    import importlib
+    B = importlib.import_module("tiktok_techjam_2026_track3_amd.build")
+
+    def unit(*lines):
+        return "\n".join(["_Z11gemm_kernelv:", *lines, ".Lfunc_end0:"])
+
+    mfma = "v_mfma_f32_16x16x32_f16 v[0:3], v[8:11], v[12:15], v[0:3] ; comment v9"
+    clean = unit("v_mov_b32_e32 v8, 0", "s_nop 1", mfma, mfma, "s_nop 15", "s_nop 1",
+                 "v_add_f32_e32 v5, v0, v1")
+    assert B.mfma_hazards(clean) == []
+    B.check_mfma_hazards("a.hip", clean)
+    close = unit("v_mov_b32_e32 v9, 0", "v_mov_b32_e32 v20, 0", mfma)
+    assert [b[1] for b in B.mfma_hazards(close)] == ["v_mov_b32_e32 v9, 0"]
+    early = unit(mfma, "s_nop 15", "v_add_f32_e32 v5, v0, v1")
+    assert B.mfma_hazards(early)
+    operand = unit(mfma, "v_mfma_f32_16x16x32_f16 v[4:7], v[0:3], v[12:15], v[4:7]")
+    assert B.mfma_hazards(operand)
+    loop = unit("v_mov_b32_e32 v9, 0", "s_nop 7", ".LBB0_1:", mfma, "s_nop 1", "v_mov_b32_e32 v10, 0",
+                "s_cbranch_scc1 .LBB0_1", "s_endpgm")
+    assert [b[1] for b in B.mfma_hazards(loop)] == ["v_mov_b32_e32 v10, 0"]
+    with pytest.raises(RuntimeError, match="wait"):
+        B.check_mfma_hazards("a.hip", close)
+
+
 def test_layernorm_cvt_argument_validation():
     """mi355_layernorm_cvt: same-dtype calls are mi355_layernorm; fp32 -> fp16 is the one
     converting pair; the checks run before any launch."""
