@@ -386,15 +386,6 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void block_head(HeadArgs p) {
   }
 }
 
-// compute units of the current device
-int cu_count() {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    return 0;
-  return cus;
-}
-
 template <typename T, int D>
 int launch_head(const HeadArgs& a, hipStream_t s) {
   constexpr int64_t BIG = 16 * 2 * 8, SMALL = 16 * 4;

@@ -2,6 +2,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <atomic>
 #include <stdint.h>
 
 #include "../../include/mi355attn.h"
@@ -283,6 +284,17 @@ MI355_DEVINL float gelu_erf(float x) {
   const float half_erfc = 0.5f * t * __builtin_amdgcn_exp2f(arg * 1.4426950408889634f);
   const float phi = x >= 0.f ? 1.0f - half_erfc : half_erfc;
   return x * phi;
+}
+
+// compute units of the current device (persistent grids), looked up once per device; 0: unknown
+inline int cu_count() {
+  static std::atomic<int> cache[64];
+  int dev = 0, n = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0) return 0;
+  if (dev < 64 && (n = cache[dev].load(std::memory_order_relaxed)) > 0) return n;
+  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+  if (dev < 64) cache[dev].store(n, std::memory_order_relaxed);
+  return n;
 }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }

@@ -928,18 +928,6 @@ int launch_gemm_splitk(const GemmArgs& a, hipStream_t stream) {
 #define MI355_GEMM_PERSIST 1
 #endif
 
-// compute units of the current device (persistent grids), looked up once per device
-int cu_count() {
-  static int cache[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0) return 0;
-  if (dev < 64 && cache[dev] > 0) return cache[dev];
-  int n = 0;
-  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-  if (dev < 64) cache[dev] = n;
-  return n;
-}
-
 template <typename T, typename TO, int BM, int BN, int WM, int WN, bool INT8>
 int launch_gemm(const GemmArgs& a, hipStream_t stream) {
   if constexpr (!INT8 && sizeof(T) == 2) {
@@ -993,25 +981,24 @@ int launch_gemm(const GemmArgs& a, hipStream_t stream) {
     const bool persist = ncu > 0 && a.K > 0 && a.K % BK == 0 && (sizeof(TO) == 2 || WM * WN > 4) && tiles > 2 * static_cast<int64_t>(ncu) && (a.K / BK) % NST == 0 &&
                          a.N % EPC_OUT == 0 && a.ldc % EPC_OUT == 0 && aligned16(a.C) &&
                          (!a.R || (a.ldr % EPC_OUT == 0 && aligned16(a.R)));
-    constexpr int PWM = WM, PWN = WN;
     // (16-bit operands; the LayerNorm fold only for the output types its tiled path takes)
     constexpr bool LNF_TO = __is_same(T, TO) || __is_same(TO, _Float16);
     const bool lnf = a.ln_stats != nullptr;
     if (persist && (LNF_TO || !lnf)) {
       if (a.kb_out) return MI355_E_UNSUPPORTED;  // the persistent epilogue has no key bounds
       if constexpr (sizeof(T) == 2 && (sizeof(TO) == 2 || WM * WN > 4)) {
-        const dim3 pgrid(static_cast<unsigned>(ncu)), pblock(PWM * PWN * 64);
+        const dim3 pgrid(static_cast<unsigned>(ncu));
         if (lnf) {
           if constexpr (LNF_TO) {
             if (gelu)
-              hipLaunchKernelGGL((gemm_kernel<T, TO, BM, BN, PWM, PWN, false, true, true, true, true>), pgrid, pblock, 0, stream, a);
+              hipLaunchKernelGGL((gemm_kernel<T, TO, BM, BN, WM, WN, false, true, true, true, true>), pgrid, block, 0, stream, a);
             else
-              hipLaunchKernelGGL((gemm_kernel<T, TO, BM, BN, PWM, PWN, false, true, false, true, true>), pgrid, pblock, 0, stream, a);
+              hipLaunchKernelGGL((gemm_kernel<T, TO, BM, BN, WM, WN, false, true, false, true, true>), pgrid, block, 0, stream, a);
           }
         } else if (gelu)
-          hipLaunchKernelGGL((gemm_kernel<T, TO, BM, BN, PWM, PWN, false, true, true, false, true>), pgrid, pblock, 0, stream, a);
+          hipLaunchKernelGGL((gemm_kernel<T, TO, BM, BN, WM, WN, false, true, true, false, true>), pgrid, block, 0, stream, a);
         else
-          hipLaunchKernelGGL((gemm_kernel<T, TO, BM, BN, PWM, PWN, false, true, false, false, true>), pgrid, pblock, 0, stream, a);
+          hipLaunchKernelGGL((gemm_kernel<T, TO, BM, BN, WM, WN, false, true, false, false, true>), pgrid, block, 0, stream, a);
         return static_cast<int>(hipGetLastError());
       }
     }
@@ -1046,8 +1033,6 @@ int launch_by_out(const GemmArgs& a, hipStream_t s) {
   switch (a.out_dtype) {
     case MI355_F16: return launch_gemm<T, _Float16, BM, BN, WM, WN, INT8>(a, s);
     case MI355_BF16: return launch_gemm<T, __bf16, BM, BN, WM, WN, INT8>(a, s);
-    // (fp32 outputs of int8 operands keep 8 waves: their unstaged GELU epilogue indexes a 128 x 128
-    // wave tile's accumulators through scratch memory)
     default: return launch_gemm<T, float, BM, BN, WM, WN, INT8>(a, s);
   }
 }
