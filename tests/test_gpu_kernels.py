@@ -160,9 +160,10 @@ def _attn_check(gpu, dtype, B, H, Sq, Sk, hd, causal, key_valid=None, packed=Fal
     # the exp2 argument s*c - m carries an fp32 rounding error relative to its largest
     # magnitude: allow 2^-22 * max|logit2| relative error on every probability
     logit2 = (tq @ tk.transpose(-2, -1)).abs().max().item() * c
-    # the kernel rounds c*q back to the input dtype: |d s*c| <= u_in * c * (|q|.|k|) per score
+    # attn_fwd_mfma rounds c*q back to the input dtype: |d s*c| <= u_in * c * (|q|.|k|) per score; the
+    # other kernels keep q as it is
     qk_abs = (tq.abs() @ tk.abs().transpose(-2, -1)).amax(dim=-1, keepdim=True).transpose(1, 2)
-    uq = UNIT[dtype] if dtype != torch.float32 else 0.0
+    uq = UNIT[dtype] if dtype != torch.float32 and hd in (32, 64, 128) else 0.0
     rel = 2 * up + 2.0 ** -18 + 2.0 ** -22 * logit2 + 2 * math.log(2) * uq * c * qk_abs
     if dtype == torch.float16 and hd in (32, 64):
         # the MFMA kernel sums a sub-tile's 32 rounded fp16 probabilities per lane in a 4-level
@@ -269,8 +270,9 @@ def test_attention_rejects_unsupported_head_dim(gpu):
         ops.attention(q, q, q)
 
 
-# head dims of the vector-ALU kernel: 8 (2 lanes per query), 16-96 (4 lanes), 192 and 256
-# (8 lanes); the benchmark's official shapes use 8, 32 and 256 (Project/shapes.json)
+# head dims beside the 64 / 128 of attn_fwd_mfma's tests: at these small sizes the vector-ALU kernel
+# (fp32: 2 lanes per query at 8, 4 at 16-96, 8 above) or attn_fwd_tiled (16-bit, but 32); the
+# benchmark's official shapes use 8, 32 and 256 (Project/shapes.json)
 VALU_HDS = [8, 16, 32, 48, 80, 96, 192, 256]
 
 
@@ -286,11 +288,10 @@ def test_attention_other_head_dims(gpu, dtype, hd, causal, S):
 @pytest.mark.parametrize("hd", [8, 32, 64, 128, 256])
 @pytest.mark.parametrize("causal", [False, True])
 def test_attention_short_keys_many_tiles(gpu, dtype, hd, causal):
-    """Up to 256 keys and at least 1024 query tiles: the vector-ALU kernel splits each tile's
-    keys over 2 waves instead of 8 (B 48, H 8, S 100: 1536 to 4992 tiles), with and without a
-    key mask, and on packed q/k/v views (the strides the model passes). fp32 head dims 64 and
-    128 take this path in production (official shapes 9 and 10); 16-bit 64 / 128 run the MFMA
-    kernel at the same shapes."""
+    """384 heads of 100 queries and keys, with and without a key mask, and on packed q/k/v views
+    (the strides the model passes): the matrix-core kernels (16-bit; fp32 32 and 64), and for fp32 the
+    vector-ALU kernel where 100 of a tile's 128 queries are too few (8, 256 and causal), which splits
+    each tile's keys over 2 waves there (up to 256 keys, at least 1024 tiles)."""
     B, S = 48, 100
     g = torch.Generator().manual_seed(hd + 7)
     mask = torch.rand(B, S, generator=g) > 0.2
@@ -304,11 +305,50 @@ def test_attention_short_keys_many_tiles(gpu, dtype, hd, causal):
 @pytest.mark.parametrize("hd", [32, 64])
 @pytest.mark.parametrize("S", [256, 257])
 def test_attention_key_split_switch_point(gpu, dtype, hd, S):
-    """Both sides of the vector-ALU kernel's 2-wave / 8-wave key split (at most 256 keys and at
-    least 1024 query tiles take 2 waves): S = 256 and S = 257 with enough tiles."""
+    """256 and 257 keys over many heads on the matrix-core kernels (the vector-ALU kernel's key split
+    at that length: test_attention_valu_key_split)."""
     B = 64 if hd == 32 else 128
     _attn_check(gpu, dtype, B, 4, S, S, hd, False, seed=S + hd)
     _attn_check(gpu, dtype, B, 4, S, S, hd, True, seed=S + hd + 1)
+
+
+@pytest.mark.parametrize("hd", [8, 16, 32, 48, 64, 80, 96, 128, 192, 256])
+@pytest.mark.parametrize("Sk", [1, 7, 256, 257])
+def test_attention_valu_key_split(gpu, hd, Sk):
+    """The vector-ALU kernel's 2-wave key split (at most 256 keys, at least 1024 query tiles: 360 heads
+    of 48 queries, too few for attn_fwd_f32) and, at 257 keys, its 8-wave one, with and without a key
+    mask, causal and on packed views."""
+    B, Sq = 90 if hd > 8 else 130, 48
+    kv = torch.rand(B, Sk, generator=torch.Generator().manual_seed(hd)) > 0.3
+    kv[:, 0] = True
+    for causal, mask in ((False, None), (False, kv), (True, kv)):
+        _attn_check(gpu, torch.float32, B, 4, Sq, Sk, hd, causal, key_valid=mask, seed=hd + Sk)
+    if Sk == 1:
+        _attn_check(gpu, torch.float32, B, 4, Sq, Sq, hd, True, packed=True, seed=hd)
+    if hd == 64:  # 200 work-groups of attn_fwd_f32, 1600 tiles here
+        _attn_check(gpu, torch.float32, 50, 4, 128, 128, hd, False, seed=3)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("hd", [192, 256])
+@pytest.mark.parametrize("S", [1, 4, 8])
+@pytest.mark.parametrize("causal", [False, True])
+def test_attention_valu_16bit_many_heads(gpu, dtype, hd, S, causal):
+    """At most 8 queries and keys of 1200 heads: the 16-bit vector-ALU instances with two waves."""
+    kv = torch.rand(300, S, generator=torch.Generator().manual_seed(hd)) > 0.3
+    kv[:, 0] = True
+    for mask in (None, kv):
+        _attn_check(gpu, dtype, 300, 4, S, S, hd, causal, key_valid=mask, seed=hd + S)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("hd", [8, 16, 48, 80, 96, 192, 256])
+@pytest.mark.parametrize("Sq", [1, 32, 33])
+def test_attention_tiled_few_queries_many_keys(gpu, dtype, hd, Sq):
+    """A few queries against thousands of keys: one wave walks them all (Sq <= 32, up to 96)."""
+    kv = torch.rand(2, 4100, generator=torch.Generator().manual_seed(hd)) > 0.3
+    for mask in (None, kv):
+        _attn_check(gpu, dtype, 2, 2, Sq, 4100, hd, False, key_valid=mask, seed=hd + Sq, qscale=2.0)
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
@@ -858,12 +898,12 @@ def test_attention_tiled_edges(gpu, dtype, hd, B, Sq, Sk, H):
                                    (64, 9), (65, 4), (80, 4), (81, 4), (65, 5)])
 def test_attention_wide_heads_both_sides_of_the_rule(gpu, dtype, hd, Sq, Sk):
     """Shapes next to each line of valu_wins_wide, with few and with many (batch, head) pairs (the
-    vector-ALU kernel's 8- and 2-wave key split), with and without a key mask."""
-    for B in (2, 300):
-        kv = torch.rand(B, Sk, generator=torch.Generator().manual_seed(Sk)) > 0.3
-        kv[:, 0] = True
-        for mask in (None, kv):
-            _attn_check(gpu, dtype, B, 4, Sq, Sk, hd, False, seed=hd + Sk, key_valid=mask)
+    vector-ALU kernel's 8- and 2-wave key split), a key mask with the former."""
+    kv = torch.rand(2, Sk, generator=torch.Generator().manual_seed(Sk)) > 0.3
+    kv[:, 0] = True
+    _attn_check(gpu, dtype, 2, 4, Sq, Sk, hd, False, seed=hd + Sk)
+    _attn_check(gpu, dtype, 2, 4, Sq, Sk, hd, False, seed=hd + Sk, key_valid=kv)
+    _attn_check(gpu, dtype, 130, 8, Sq, Sk, hd, False, seed=hd + Sk)
 
 
 @pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
@@ -901,6 +941,28 @@ def test_attention_f32_mfma_edges(gpu, hd, B, Sq, Sk):
         if Sq == Sk:
             _attn_check(gpu, torch.float32, B, 2, Sq, Sk, hd, True, seed=hd + 7, key_valid=mask,
                         packed=True)
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("hd", [8, 48, 64, 256])
+def test_attention_f32_nonfinite_rows_stay_in_their_queries(gpu, hd, bad):
+    """As for attn_fwd_tiled: a non-finite element of one query row, or of a masked-out key's K row,
+    reaches no other row."""
+    ops = _ops()
+    B, S = 130, 128
+    q, k, v = (_rand((B, S, 2, hd), torch.float32, s).to(gpu) for s in (1, 2, 3))
+    kv = torch.ones(B, S, dtype=torch.bool, device=gpu)
+    kv[0, 66] = False
+    ref = ops.attention(q, k, v, key_valid=kv)
+    q2, k2 = q.clone(), k.clone()
+    q2[0, 5, 0, 1] = bad
+    k2[0, 66, :, 0] = bad
+    out = ops.attention(q2, k2, v, key_valid=kv)
+    keep = torch.ones(S, dtype=torch.bool, device=gpu)
+    keep[5] = False
+    assert torch.equal(out[:, keep], ref[:, keep])
+    assert torch.equal(out[:, 5, 1], ref[:, 5, 1])
+    assert torch.equal(out[1:], ref[1:])
 
 
 @pytest.mark.parametrize("hd,n,Sq,Sk,causal", [
@@ -978,6 +1040,50 @@ def test_linear_ragged_k(gpu, dtype, M, N, K):
     ref = a64 @ w64.T + b.double()
     bound = UNIT[dtype] * ref.abs() + 4 * K * 2.0 ** -24 * (a64.abs() @ w64.abs().T) + 1e-7
     assert _report("linear", (out - ref).abs(), bound) <= 1.0
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,K", [(8300, 64), (16500, 72), (33000, 128), (66000, 40)])
+def test_linear_row_pitch_beyond_the_direct_loader(gpu, dtype, N, K):
+    """Rows more than 8 MiB apart take the register-staged loader, at each of its tiles: 64 x 64,
+    128 x 128 and (16-bit, the widest) where 256 x 256 would be taken. Plain, with the GELU epilogue
+    and with a LayerNorm folded in."""
+    ops = _ops()
+    M, es = 64, torch.finfo(dtype).bits // 8
+    pitch = (1 << 23) // es + 16 // es
+    buf = torch.empty(M * pitch, dtype=dtype, device=gpu)
+    x = buf.as_strided((M, K), (pitch, 1))
+    a = _rand((M, K), dtype, 1)
+    x.copy_(a)
+    w = _rand((N, K), dtype, 2, scale=K ** -0.5)
+    b = _rand((N,), torch.float32, 3, scale=0.1)
+    print(f"pitch dtype={dtype} N={N} K={K}", flush=True)
+    wg, bg = w.to(gpu), b.to(gpu)
+    out = ops.linear(x, wg, bg).cpu().double()
+    a64, w64 = a.double(), w.double()
+    ref = a64 @ w64.T + b.double()
+    mag = a64.abs() @ w64.abs().T
+    bound = UNIT[dtype] * ref.abs() + 4 * K * 2.0 ** -24 * mag + 1e-7
+    assert _report("linear", (out - ref).abs(), bound) <= 1.0
+    # the same rows close together: the LDS-DMA loader, whose products run in the same order
+    near = a.to(gpu)
+    assert torch.equal(ops.linear(x, wg, bg, gelu=True), ops.linear(near, wg, bg, gelu=True))
+    if dtype != torch.bfloat16:
+        col = wg.float().sum(1)
+        assert torch.equal(ops.layernorm_linear(x, wg, col, bg), ops.layernorm_linear(near, wg, col, bg))
+
+
+def test_gemm_i8_row_pitch_beyond_the_direct_loader(gpu):
+    """int8 rows longer than 8 MiB (contiguous, so K is the pitch): bit for bit."""
+    ops = _ops()
+    M, N, K = 20, 24, (1 << 23) + 48
+    g = torch.Generator(device=gpu).manual_seed(4)
+    a, w = (torch.randint(-1, 2, (n, K), generator=g, device=gpu, dtype=torch.int8) for n in (M, N))
+    acc = torch.empty(M, N, dtype=torch.int32, device=gpu)
+    print("pitch int8", flush=True)
+    ops.linear_i8(a, w, torch.ones(M, device=gpu), torch.ones(N, device=gpu), acc_out=acc, want_out=False)
+    ref = sum(a[:, i:i + (1 << 20)].float() @ w[:, i:i + (1 << 20)].float().T for i in range(0, K, 1 << 20))
+    assert torch.equal(acc.float(), ref)  # (partial sums below 2^23: exact)
 
 
 @pytest.mark.parametrize("M,N,K", [(2100, 1100, 16), (4100, 4360, 144), (1100, 3000, 272)])
