@@ -343,6 +343,24 @@ def test_attention_valu_16bit_many_heads(gpu, dtype, hd, S, causal):
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("hd", [8, 16, 48, 80, 96, 192, 256])
+@pytest.mark.parametrize("S,causal", [(130, True), (700, False), (700, True)])
+def test_attention_tiled_error_is_the_outputs_rounding(gpu, dtype, hd, S, causal):
+    """attn_fwd_tiled multiplies probabilities of two terms of the input type: what is left of the
+    error against fp64 is the rounding of its output, and 2^-16 (bf16) or less of the probabilities.
+    (Probabilities rounded once add a fifth to half of that again.)"""
+    ops = _ops()
+    q, k, v = (_rand((2, S, 2, hd), dtype, hd + S + i) for i in range(3))
+    out = ops.attention(q.to(gpu), k.to(gpu), v.to(gpu), causal=causal).cpu().double()
+    ref = OA.attention_core(*(t.double().transpose(1, 2) for t in (q, k, v)), hd ** -0.5, causal,
+                            None).transpose(1, 2)
+    rounding = float((ref.to(dtype).double() - ref).norm())
+    err = float((out - ref).norm())
+    print(f"tiled error {dtype} hd={hd} S={S} causal={causal}: {err / rounding:.4f} of the rounding", flush=True)
+    assert err <= 1.05 * rounding
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("hd", [8, 16, 48, 80, 96, 192, 256])
 @pytest.mark.parametrize("Sq", [1, 32, 33])
 def test_attention_tiled_few_queries_many_keys(gpu, dtype, hd, Sq):
     """A few queries against thousands of keys: one wave walks them all (Sq <= 32, up to 96)."""
@@ -894,8 +912,9 @@ def test_attention_tiled_edges(gpu, dtype, hd, B, Sq, Sk, H):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("hd", [192, 256])
 @pytest.mark.parametrize("Sq,Sk", [(1, 9), (8, 32), (1, 33), (8, 112), (8, 113), (8, 160), (8, 161),
-                                   (9, 33), (16, 48), (16, 49), (17, 33), (33, 10), (48, 11), (64, 8),
-                                   (64, 9), (65, 4), (80, 4), (81, 4), (65, 5)])
+                                   (8, 144), (8, 145),
+                                   (9, 33), (16, 48), (16, 49), (17, 33), (33, 10), (48, 11), (64, 10),
+                                   (64, 11), (65, 4), (80, 4), (81, 4), (65, 5)])
 def test_attention_wide_heads_both_sides_of_the_rule(gpu, dtype, hd, Sq, Sk):
     """Shapes next to each line of valu_wins_wide, with few and with many (batch, head) pairs (the
     vector-ALU kernel's 8- and 2-wave key split), a key mask with the former."""

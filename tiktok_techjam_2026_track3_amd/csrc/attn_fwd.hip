@@ -1628,15 +1628,15 @@ int64_t redo_flag_bytes(int64_t B, int64_t H, int64_t S_q, int64_t head_dim) {
 // than a mostly empty tile of attn_fwd_tiled (vector-ALU -> tiled, us, at 256 unless said otherwise).
 // Up to 32 queries that one has a 32-key tile on one wave (8192 heads of 4 and 4: 32 -> 43; of 16: 103
 // -> 60) or, beyond 32 keys, 64-key tiles in the whole LDS for one busy wave of four (2048 heads of 8
-// queries and 33 keys 32 -> 54; 12000 heads and 112 keys 1.2, at 192 1.1, 128 keys 0.96 there; 160 keys
-// 1.11, but 0.84 of the time for 256 heads; 16 queries and 48 keys 1.06, 64 0.74); beyond 32 queries a
-// 128-query work-group (2048 heads of 33 queries and 8 keys 46 -> 58, 12000 of 12 keys 0.97; 64 and 8
-// keys 70 -> 75, 12 keys 0.74; 80 and 4 keys at 192 1.12, 96 0.85).
+// queries and 33 keys 32 -> 54; 12000 heads and 112 keys 1.2, 160 keys 1.11, but 0.84 of the time for
+// 256 heads; at 192 2048 heads and 130 keys 81 -> 89; 16 queries and 48 keys 1.06, 64 0.74); beyond 32
+// queries a 128-query work-group (2048 heads of 33 queries and 8 keys 46 -> 58; at 192 16384 heads of 64
+// and 9 keys 665 -> 781, 2048 heads and 16 keys 0.7; 80 and 4 keys 1.12, 96 0.85).
 bool valu_wins_wide(int64_t hd, int64_t pairs, int64_t S_q, int64_t S_k) {
-  if (S_q <= 8) return S_k <= 8 || (S_k > 32 && S_k <= (hd == 256 && pairs >= 1024 ? 160 : 112));
+  if (S_q <= 8) return S_k <= 8 || (S_k > 32 && S_k <= (pairs < 1024 ? 112 : hd == 256 ? 160 : 144));
   if (S_q <= 16) return S_k > 32 && S_k <= 48;
   if (S_q <= 32) return false;
-  return S_k <= (S_q <= 48 ? 10 : S_q <= 64 ? 8 : S_q <= 80 ? 4 : 0);
+  return S_k <= (S_q <= 64 ? 10 : S_q <= 80 ? 4 : 0);
 }
 
 int attn_fwd_impl(int dtype, const void* Q, const void* K, const void* V, void* O, int64_t B,

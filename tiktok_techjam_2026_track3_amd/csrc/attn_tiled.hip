@@ -9,12 +9,17 @@
 //     whose rows past hd hold garbage that is never stored, and rows keep their natural LDS pitch
 //     with a swizzle only where that pitch would collide (swz_row);
 //   * Q stays as it is in memory and the scores are scaled in fp32 after the MFMA (one FMA per
-//     score, folded with the running max), so nothing is rounded that the fp32 vector-ALU kernel
-//     it takes over from did not round: the probabilities, once, to the input type. The row sums
-//     add the rounded probabilities in fp32;
-//   * measured against that kernel (fp16): B4 H8 S2048 hd 80 1433 -> 60 us (724 TFLOP/s), hd 96
-//     1607 -> 62 (830), hd 256 4640 -> 137 (1002), hd 16 336 -> 33; causal B64 H4 S128 hd 256 81 ->
-//     22; the last are bound by the exponentials, the wide ones by MFMAs and power;
+//     score, folded with the running max);
+//   * the probabilities enter P · V as the sum of two terms of the input type (22 or 16 bits), the row
+//     sums add them in fp32. The fp32 vector-ALU kernel this one takes over from rounded them once, but
+//     relative to eight key ranges' exact running maxima, whose keys it met as exactly 1; rounded
+//     once here, relative to one lazily moved maximum, the results' error against 64 bits was 0-5%
+//     larger over attention blocks and cores of 34-17000 tokens, 8-15% for N(0, 1) scores alone; with
+//     the second term it is 0.75-1.0 of that kernel's. The second term costs 28-50% of long sweeps
+//     (an exact running max 4-12%, for half of the loss);
+//   * measured against that kernel (fp16): B4 H8 S2048 hd 80 1430 -> 78 us, hd 96 1603 -> 83, hd 256
+//     4613 -> 181, hd 16 313 -> 41; causal B64 H4 S128 hd 256 74 -> 21; the narrow ones are bound by
+//     the exponentials, the wide ones by MFMAs and power;
 //   * causal and key masks are run-time: a tile is masked element by element only where it crosses
 //     the diagonal, the end or an invalid key (a ballot of its 64 mask bytes).
 #include "attn.h"
@@ -38,20 +43,6 @@ MI355_DEVINL int swz_row(int r) {
     return 0;
   else
     return (r >> 4) & 1;
-}
-
-MI355_DEVINL float sum8(f16x8 f, float acc) {
-  const f16x2 one = {(_Float16)1.0f, (_Float16)1.0f};
-#pragma unroll
-  for (int r = 0; r < 4; ++r) acc = __builtin_amdgcn_fdot2(f16x2{f[2 * r], f[2 * r + 1]}, one, acc, false);
-  return acc;
-}
-MI355_DEVINL float sum8(bf16x8 f, float acc) {
-  const bf16x2 one = {(__bf16)1.0f, (__bf16)1.0f};
-#pragma unroll
-  for (int r = 0; r < 4; ++r)
-    acc = __builtin_amdgcn_fdot2_f32_bf16(bf16x2{f[2 * r], f[2 * r + 1]}, one, acc, false);
-  return acc;
 }
 
 // NW waves of QG groups of 32 queries of one (batch, head). LAP: K or V rows that overlap (a stride
@@ -284,27 +275,42 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_fwd_tiled(AttnArgs p) {
         gate[n] = grow ? mx + 8.f : gate[n];
       }
     }
-    frag pf[QG][U][2];
+    // probabilities as two terms of the input type, hi = p rounded and lo = the rest rounded
+    frag pf[2][QG][U][2];
 #pragma unroll
     for (int n = 0; n < QG; ++n)
 #pragma unroll
       for (int u = 0; u < U; ++u)
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh) {
+          float e[8];
+#pragma unroll
+          for (int r = 0; r < 8; ++r) {
+            e[r] = fast_exp2(__builtin_fmaf(s[n][u][8 * hh + r], p.c, -mu[n]));
+            pf[0][n][u][hh][r] = from_f32<T>(e[r]);
+          }
 #pragma unroll
           for (int r = 0; r < 8; ++r)
-            pf[n][u][hh][r] = from_f32<T>(fast_exp2(__builtin_fmaf(s[n][u][8 * hh + r], p.c, -mu[n])));
-          lsum[n] = sum8(pf[n][u][hh], lsum[n]);
+            pf[1][n][u][hh][r] = from_f32<T>(__builtin_fmaf(to_f32(pf[0][n][u][hh][r]), -1.0f, e[r]));
+          lsum[n] += ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
         }
+    // two row blocks at a time, so that an accumulator's MFMAs do not follow each other
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+    for (int m0 = 0; m0 < MT; m0 += 2)
 #pragma unroll
       for (int u = 0; u < U; ++u)
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh) {
-          const frag vf = vfrag(st, mt, t0 + u, hh);
+          frag vf[2];
 #pragma unroll
-          for (int n = 0; n < QG; ++n) oacc[n][mt] = MF::mma(vf, pf[n][u][hh], oacc[n][mt]);
+          for (int m = 0; m < 2 && m0 + m < MT; ++m) vf[m] = vfrag(st, m0 + m, t0 + u, hh);
+#pragma unroll
+          for (int l = 0; l < 2; ++l)
+#pragma unroll
+            for (int m = 0; m < 2 && m0 + m < MT; ++m)
+#pragma unroll
+              for (int n = 0; n < QG; ++n)
+                oacc[n][m0 + m] = MF::mma(vf[m], pf[l][n][u][hh], oacc[n][m0 + m]);
         }
   };
 
