@@ -12,7 +12,8 @@
 //
 // Measured against the vector-ALU kernel (B4 H8 S2048): hd 8 191 -> 89 us, hd 32 443 -> 174, hd 64
 // 974 -> 290 (118 TFLOP/s of the 157 the fp32 MFMAs have), hd 256 3951 -> 1481; causal B512 H16
-// S128 hd 8 187 -> 80; the errors against 64 bits are the same or smaller. The narrow heads are
+// S128 hd 8 187 -> 80; the errors against 64 bits are smaller but for a
+// few short causal ranges (see the score chains below). The narrow heads are
 // bound by the exponentials and by O^T's padding to 16 rows, the wide ones by the MFMAs.
 #include "attn.h"
 
@@ -135,7 +136,8 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_fwd_f32(AttnArgs p) {
   auto compute = [&](const int j, const int st, const uint64_t vbits) MI355_LAMBDA_INLINE {
     const float* kt = reinterpret_cast<const float*>(&lds[st * TILE]);
     const float* vt = reinterpret_cast<const float*>(&lds[(2 + st) * TILE]);
-    f32x4 s[QG][KB];
+    constexpr bool ODD = KS >= 4;
+    f32x4 s[QG][KB], odd[QG][ODD ? KB : 1];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       float kf[KB][KE];
@@ -153,20 +155,36 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_fwd_f32(AttnArgs p) {
           for (int e = 0; e < KE; ++e) kf[kb][e] = v[e];
         }
       }
-      // a fragment's 16 dims are summed on their own and then added (below: why)
+      // a fragment's 16 dims are summed on their own and then added (below: why), from hd 64 on even
+      // and odd fragments apart, and the halves of hd 16's one fragment. In one chain the scores of 300
+      // causal keys were 2-12% further off than the vector-ALU kernel's, now -5 to 2% (1000 keys and
+      // more -5 to -23% either way). Halves at every hd: -1 to -5%, for 10-20% of the time at 48, 64.
+      constexpr bool HALVES = KE == 4 && KS == 1;
 #pragma unroll
       for (int n = 0; n < QG; ++n) {
-        f32x4 d[KB];
+        f32x4 d[2][KB];
 #pragma unroll
-        for (int kb = 0; kb < KB; ++kb) d[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int kb = 0; kb < KB; ++kb) d[0][kb] = d[1][kb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int e = 0; e < KE; ++e)
 #pragma unroll
-          for (int kb = 0; kb < KB; ++kb)
-            d[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[kb][e], qf[n][ks][e], d[kb], 0, 0, 0);
+          for (int kb = 0; kb < KB; ++kb) {
+            f32x4& to = d[HALVES ? e / 2 : 0][kb];
+            to = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[kb][e], qf[n][ks][e], to, 0, 0, 0);
+          }
 #pragma unroll
-        for (int kb = 0; kb < KB; ++kb) s[n][kb] = ks == 0 ? d[kb] : s[n][kb] + d[kb];
+        for (int kb = 0; kb < KB; ++kb) {
+          const f32x4 sum = HALVES ? d[0][kb] + d[1][kb] : d[0][kb];
+          f32x4& to = ODD && ks % 2 ? odd[n][kb] : s[n][kb];
+          to = ks < (ODD ? 2 : 1) ? sum : to + sum;
+        }
       }
+    }
+    if constexpr (ODD) {
+#pragma unroll
+      for (int n = 0; n < QG; ++n)
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) s[n][kb] += odd[n][kb];
     }
     const int k0 = j * BN;
     if (vbits != ~0ull || k0 + BN > Sk || (CAUSAL && k0 + BN - 1 > q_wave)) {
@@ -356,7 +374,8 @@ int launch_hd(const AttnArgs& a, bool causal, hipStream_t s) {
 //     keys at hd 8 82 -> 149; 512 heads of 65 queries 241 -> 270, 800 of them 0.72 of the time);
 //   * up to hd 64: fewer than 64 keys, or 32 in full tiles of four waves (hd 32, 2048 heads of 64
 //     queries and 16 keys 0.69 of its speed; 129 queries and 32 keys 0.84, 64 keys 1.4);
-//   * above: up to 256 keys (where the other kernel's key split is the cheaper one of two waves) it
+//   * above: up to 256 keys (where the other kernel's key split is the cheaper one of two waves; above
+//     hd 128 223: 256 heads of 65 queries and 256 keys at 256 141 -> 105) it
 //     has to fill two thirds of its tiles: 512 heads of 128 queries and 64 keys at hd 80 0.70 of the
 //     time, of 129 queries 0.90, of 64 queries 0.87, at 800 heads 0.86, 1.15 and 1.24; one key 2-4;
 //   * causal, up to 256 keys: half of those are skipped by 16-query steps there, by tiles here, so
@@ -389,7 +408,7 @@ bool mi355_internal_attn_f32_wins(const AttnTiledCall& call) {
     return hd == 8 || keys >= 64 || filled(90);
   }
   if (hd <= 64) return keys >= 64 || (keys >= 32 && filled(90) && !two_waves);
-  if (keys > 256) return true;
+  if (keys > (hd > 128 ? 223 : 256)) return true;
   if (keys < 64 || (hd <= 128 && two_waves)) return false;
   const int64_t bn = hd > 128 ? 32 : 64, padded = (keys + bn - 1) / bn * bn;
   return 100 * a.Sq * keys >= (hd > 128 ? 70 : 66) * tiles * bm * padded;
