@@ -347,7 +347,7 @@ class SelfAttention(nn.Module):
         """norm, QKV projection and attention of ``forward_residual``: ``(ctx [T, d], x [T, d],
         row_valid, W_o, b_o)``, what the out projection and the residual need. ``fused``: narrow
         fp32 models on fp16 operands run norm and projection as one launch (``ops.block_head``:
-        1 280 000 x 128 rows 590 -> 370 us), so no "norm" / "qkv" stages are marked."""
+        1 280 000 x 128 rows 590 -> 385 us), so no "norm" / "qkv" stages are marked."""
         B, S = self._check_input(x)
         d = self.d_model
         if tuple(norm.normalized_shape) != (d,):

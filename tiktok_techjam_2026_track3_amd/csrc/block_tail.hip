@@ -16,8 +16,8 @@
 // separate launches (where the out projection is not the split-K kernel's); one GELU output in
 // millions differs by an fp16 step: there the compiler rounds x Phi(x) to fp16 at once
 // (v_fma_mixlo_f16), here in pairs after fp32, and forcing the former cost 3%. [1280000, 128]
-// fp32: the four launches 1425 us, this one 430; the official 4-layer model over 10 000 sequences
-// 10.42 -> 5.49 ms, over 64 0.210 -> 0.162.
+// fp32: the four launches 1425 us, this one 428; the official 4-layer model over 10 000 sequences
+// 10.36 -> 5.49 ms, over 64 0.210 -> 0.146.
 #include <type_traits>
 
 #include "common.h"
@@ -271,8 +271,8 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void block_tail(TailArgs p) {
 // The block's other end: qkv = fp16(norm1(x) W_qkv^T + b), the norm's output rounded to fp16 in
 // registers, W_qkv [3 D, D] resident in LDS. Reads a row once and writes its 3 D features; as
 // LayerNorm kernel and projection, the normalised rows are written and read in between
-// ([1280000, 128] fp32: 195 + 395 us against 372; the official model over 10 000 sequences 5.49 ->
-// 4.54 ms).
+// ([1280000, 128] fp32: 195 + 395 us against 385; the official model over 10 000 sequences 5.49 ->
+// 4.59 ms).
 struct HeadArgs {
   const void* x;            // [M, D], row stride ldx
   const void *gamma, *beta;  // [D] of x's type, nullable

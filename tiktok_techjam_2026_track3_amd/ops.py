@@ -378,7 +378,8 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: Optional[t
 # d_model that block_head takes: the packed QKV weight resident in LDS
 BLOCK_HEAD_SIZES = frozenset((32, 64, 128))
 # ... and the rows from which it pays: every CU's work-group stages the whole weight (96 KB at d
-# 128) for its rows, which on 8192 rows cost more than the launch saved (4-layer model 162 -> 178 us)
+# 128) for its rows, which on 8192 rows cost more than the launch saved (4-layer model 162 -> 178 us);
+# from 65536 rows on a work-group per CU walks them (a layer of d 128: 108 -> 73 us there)
 BLOCK_HEAD_MIN_ROWS = 65536
 
 

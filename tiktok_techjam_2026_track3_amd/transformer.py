@@ -120,7 +120,7 @@ def _takes_tail(block: nn.Module, x: torch.Tensor) -> bool:
     """Whether the block's out projection, norm2 and FFN run as one launch (``ops.block_tail``):
     fp16 operands and attention core, norm2 as its own rounding step (not folded into ffn_in) and
     weights that fit the kernel together. There the separate launches are bound by their passes
-    over memory and, at small batches, by their number: 1 280 000 x 128 fp32 rows 1425 -> 430 us."""
+    over memory and, at small batches, by their number: 1 280 000 x 128 fp32 rows 1425 -> 428 us."""
     attn = block.attention
     # first what most blocks fail: a small layer's forward is bound by its host code
     return (not attn.folds_norm(x.dtype, x.numel())
@@ -152,7 +152,8 @@ def block_forward(block: nn.Module, x: torch.Tensor, valid_token_mask: Optional[
     normalised activation is written. ``marks(stage)`` is called before each launch ("qkv",
     "attn", "out", "ffn_in", "ffn_out"; unfolded, "norm" and "norm2" before the LayerNorm
     kernels; the int8 block adds its quantisation launches) and after the last ("end"); without it,
-    narrow blocks on fp16 operands run everything after the attention as one launch (``_takes_tail``).
+    narrow blocks on fp16 operands run everything after the attention as one launch (``_takes_tail``),
+    so the stages of such a block are those of the separate launches, not of its forward.
     ``keep`` (a dict) receives the int8 block's intermediates."""
     mark = marks or (lambda _stage: None)
     attn = block.attention
